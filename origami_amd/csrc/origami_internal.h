@@ -34,6 +34,36 @@ inline unsigned grid_for(int64_t work, int64_t per_block, int64_t cap) {
 }
 
 // ---------------------------------------------------------------------------
+// Symbol runs (origami_runs.hip)
+// ---------------------------------------------------------------------------
+
+// `count` symbols that are consecutive bytes of the symbol tensor from `symbol`, and
+// consecutive in the stream from byte `byte` of it.
+struct SymbolRun {
+  int64_t symbol, byte, count;
+};
+
+constexpr int kMaxSymbolRuns = 8;  // runs of one launch (kernel arguments)
+
+// The runs of a chunk plan whose chunks are all memory runs of the symbol tensor, of
+// one width; chunks that follow each other in memory and, on a byte, in the stream
+// are one run.  Returns their number, or 0 where the plan is not such runs, or more
+// than kMaxSymbolRuns.
+int collect_symbol_runs(const int64_t* offsets, const int64_t* bits, const int64_t* specs,
+                        int64_t n, int64_t stride_token, int64_t stride_head,
+                        int64_t stride_channel, SymbolRun (&runs)[kMaxSymbolRuns]);
+
+int launch_unpack_runs(const uint8_t* flat, int64_t flat_bytes, const SymbolRun* runs, int nrun,
+                       int bits, uint8_t* symbols, hipStream_t stream);
+
+// Whether every run's symbols and stream bytes start on dwords, as the packer needs.
+bool pack_runs_aligned(const uint8_t* symbols, const uint8_t* flat, const SymbolRun* runs,
+                       int nrun);
+
+int launch_pack_runs(const uint8_t* symbols, const SymbolRun* runs, int nrun, int bits,
+                     uint8_t* flat, hipStream_t stream);
+
+// ---------------------------------------------------------------------------
 // Device helpers shared by the row kernels
 // ---------------------------------------------------------------------------
 

@@ -2684,6 +2684,21 @@ int origami_unpack_canonical_storage_chunks(
   const bool rows_layout = st.channel == 1 && C % 16 == 0 && st.token % 16 == 0 &&
                            st.head % 16 == 0 && aligned16(output) && T >= 16 &&
                            H * C <= kMaxPlaneTable;
+  // Chunks that are memory runs of the tensor (plain bit streams, token-fastest
+  // tensors): 16-byte lanes and no plan.  33.5M symbols of one 5-bit stream: 84.6 us
+  // through the generic kernel and its fill, 11.7 us (4.6 TB/s) here.
+  SymbolRun runs[kMaxSymbolRuns];
+  const int nrun = rows_layout ? 0
+                               : collect_symbol_runs(chunk_offsets, bits_per_chunk, chunk_specs,
+                                                     num_chunks, st.token, st.head, st.channel,
+                                                     runs);
+  if (nrun > 0) {
+    // bytes that no chunk covers are 0
+    if (nrun != 1 || runs[0].symbol != 0 || runs[0].count != total)
+      if (int rc2 = launch_fill_zero(output, output_bytes, stream)) return rc2;
+    return launch_unpack_runs(flat_chunks, flat_bytes, runs, nrun,
+                              static_cast<int>(bits_per_chunk[0]), output, stream);
+  }
   std::shared_ptr<const Plan> plan;
   rc = get_plan(chunk_offsets, bits_per_chunk, chunk_specs, num_chunks, T, H, C, rows_layout, &plan);
   if (rc) return rc;
@@ -2739,6 +2754,17 @@ int origami_pack_canonical_storage_chunks(
   const bool rows_layout = st.channel == 1 && C % 16 == 0 && st.token % 16 == 0 &&
                            st.head % 16 == 0 && aligned16(symbols) && T >= 16 &&
                            H * C <= kMaxPlaneTable;
+  // Memory runs, as in the unpack: the two symbol streams and the stored payload of a
+  // 16384-token CacheGen save took 193 us more through the generic kernel (572 against
+  // 380 us for the whole save).
+  SymbolRun runs[kMaxSymbolRuns];
+  const int nrun = rows_layout ? 0
+                               : collect_symbol_runs(chunk_offsets, bits_per_chunk, chunk_specs,
+                                                     num_chunks, st.token, st.head, st.channel,
+                                                     runs);
+  if (nrun > 0 && pack_runs_aligned(symbols, flat_chunks, runs, nrun))
+    return launch_pack_runs(symbols, runs, nrun, static_cast<int>(bits_per_chunk[0]), flat_chunks,
+                            stream);
   std::shared_ptr<const Plan> plan;
   rc = get_plan(chunk_offsets, bits_per_chunk, chunk_specs, num_chunks, T, H, C, rows_layout, &plan);
   if (rc) return rc;
