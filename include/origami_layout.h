@@ -385,6 +385,50 @@ int origami_kivi_dequantize_to_kv_cache(
     int64_t block_size, const int64_t* block_ids, int64_t block_count,
     int64_t tokens, int64_t heads, int64_t head_dim, origami_stream_t stream);
 
+/* ---------------------------------------------------------------------------
+ * Fused quantized saves (CacheGen, KIVI): the counterparts of the restores
+ * above.  kv is a K/V tensor of dtype FLOAT16, BFLOAT16 or FLOAT32 whose
+ * element (half, token t, head h, dim d) is at half * strides[0] +
+ * (t / strides[4]) * strides[1] + (t % strides[4]) * strides[2] +
+ * h * strides[3] + d (strides: host, [5], in elements; strides[4] is the
+ * token count of a block).  Both return ORIGAMI_ERR_UNSUPPORTED, with nothing
+ * launched, unless kv is 16-byte aligned and head_dim and the strides are
+ * multiples of 8.
+ * ------------------------------------------------------------------------- */
+
+/*
+ * CacheGen quantize + bit packing (cachegen_adapter.py:246-340 of the
+ * reference).  Writes into `payload` the key symbols at key_bits from byte 0,
+ * the value symbols at value_bits from value_offset (token-major, LSB-first),
+ * and the float16 per-token maxima from key_max_offset and value_max_offset
+ * (even).  A byte between the value stream and the maxima is written as 0.
+ * key_bits = value_bits = 8 is the structured format.  At most 4096 channels
+ * (else ORIGAMI_ERR_UNSUPPORTED).
+ */
+int origami_cachegen_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t heads,
+                              int64_t head_dim, const int64_t* strides, int64_t key_bits,
+                              int64_t value_bits, int64_t key_bins, int64_t value_bins,
+                              uint8_t* payload, int64_t payload_bytes, int64_t value_offset,
+                              int64_t key_max_offset, int64_t value_max_offset,
+                              origami_stream_t stream);
+
+/*
+ * KIVI quantize + packing in KIVI's container (kivi_adapter.py:229-450 of the
+ * reference; 3-bit symbols one per nibble).  offsets (host, [8]) are the
+ * payload offsets of the key stream, value stream, key scale, key zero, value
+ * scale, value zero, key sink and value sink, in that order and without gaps
+ * other than single bytes, which are written as 0.  sink_tokens < tokens;
+ * group_size 16, 32, 64 or 128 (else ORIGAMI_ERR_UNSUPPORTED).  workspace
+ * holds 2 * heads * head_dim * (tokens - sink_tokens) bytes and is used unless
+ * tokens - sink_tokens is a multiple of 16 and the payload and its value
+ * stream are 16-byte aligned (it may be null then).
+ */
+int origami_kivi_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t heads,
+                          int64_t head_dim, const int64_t* strides, int64_t bits,
+                          int64_t group_size, int64_t sink_tokens, uint8_t* payload,
+                          int64_t payload_bytes, const int64_t* offsets, uint8_t* workspace,
+                          int64_t workspace_bytes, origami_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -63,6 +63,10 @@ _SIGNATURES: dict[str, list] = {
     "origami_kivi_dequantize_to_kv_cache": [
         _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p,
         _i64, _p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _p],
+    "origami_cachegen_quantize": [
+        _p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _p],
+    "origami_kivi_quantize": [
+        _p, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _p, _p, _i64, _p],
 }
 
 EXPORTED_SYMBOLS = ("origami_last_error", "origami_restore_plan_destroy",

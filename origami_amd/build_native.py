@@ -14,7 +14,8 @@ from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 REPO = PKG.parent
-SOURCES = [PKG / "csrc" / f"origami_{name}.hip" for name in ("layout", "dequant", "runs")]
+SOURCES = [PKG / "csrc" / f"origami_{name}.hip" 
+           for name in ("layout", "dequant", "runs", "quantize")]
 INCLUDE = REPO / "include"
 LIB_DIR = PKG / "_lib"
 LIB_PATH = LIB_DIR / "liborigami_layout.so"

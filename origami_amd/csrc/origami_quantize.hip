@@ -1,0 +1,623 @@
+// origami_quantize.hip -- MI355X (gfx950) kernels for the quantized saves: one layer's
+// K/V read once and its CacheGen or KIVI payload written once (the quantizers of the
+// reference's cachegen_adapter.py:246-340 and kivi_adapter.py:229-450, which are chains
+// of float32 tensor operations).
+//
+// Arithmetic is that of the tensor expressions, operation by operation in binary32
+// without contraction, so payloads are the same bytes: a scalar divided by a tensor is
+// the tensor's reciprocal times the scalar, a tensor divided by a scalar is the tensor
+// times the scalar's reciprocal, and a minimum or maximum with a NaN is a NaN (whose
+// symbols are 0).  The K/V tensor may have any of the layouts the adapters accept: head_dim
+// is its fastest axis, everything else is a stride (KvStrides).
+//
+// HBM bounds both: 4 bytes read and b / 4 bytes written per (K, V) pair of 16-bit
+// values.  16384 tokens of 8 heads x 128, bf16, with the copy of the payload into its
+// stored chunks: CacheGen 573 -> 30.8 us, KIVI (2 bits) 1032 -> 61.0 us.
+#include <hip/hip_runtime.h>
+
+#include <stdint.h>
+
+#include "origami_internal.h"
+#include "origami_layout.h"
+
+using namespace origami_internal;
+
+namespace {
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4u __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kQThreads = 256;
+constexpr int kQWaves = kQThreads / 64;
+
+// Element strides of a K/V tensor: element (half, token t, head h, dim d) is at
+// half * half + (t / block_tokens) * block + (t % block_tokens) * token + h * head + d.
+struct KvStrides {
+  int64_t half, block, token, head;
+  uint32_t block_tokens;
+};
+
+__device__ __forceinline__ int64_t token_offset(const KvStrides& s, uint32_t t) {
+  const uint32_t blk = t / s.block_tokens;
+  return static_cast<int64_t>(blk) * s.block +
+         static_cast<int64_t>(t - blk * s.block_tokens) * s.token;
+}
+
+// Eight consecutive elements as binary32: 16 bytes of a 16-bit type, 32 of float32.
+template <int DT>
+struct Eight {
+  static constexpr int kWords = DT == ORIGAMI_DTYPE_FLOAT32 ? 8 : 4;
+  uint32_t w[kWords];
+
+  __device__ __forceinline__ void load(const void* base, int64_t element) {
+    const u32x4* src = reinterpret_cast<const u32x4*>(
+        static_cast<const uint8_t*>(base) + element * (kWords / 2));
+#pragma unroll
+    for (int i = 0; i < kWords / 4; ++i) {
+      const u32x4 x = __builtin_nontemporal_load(src + i);
+      w[4 * i] = x.x;
+      w[4 * i + 1] = x.y;
+      w[4 * i + 2] = x.z;
+      w[4 * i + 3] = x.w;
+    }
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) w[i] = 0;
+  }
+  __device__ __forceinline__ float get(int i) const {
+    if constexpr (DT == ORIGAMI_DTYPE_FLOAT32) {
+      return __builtin_bit_cast(float, w[i]);
+    } else if constexpr (DT == ORIGAMI_DTYPE_BFLOAT16) {
+      return __builtin_bit_cast(float, i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
+    } else {
+      return static_cast<float>(
+          __builtin_bit_cast(_Float16, static_cast<uint16_t>(w[i >> 1] >> (16 * (i & 1)))));
+    }
+  }
+};
+
+__device__ __forceinline__ uint16_t half_bits(float v) {
+  asm("" : "+v"(v));  // an already rounded binary32 value (no fused convert)
+  return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
+}
+
+// ---------------------------------------------------------------------------
+// CacheGen
+// ---------------------------------------------------------------------------
+
+struct CacheGenQuantParams {
+  const void* kv;
+  KvStrides s;
+  uint32_t tokens;
+  int32_t row_lanes;   // lanes of a token row: a power of two, at most 64
+  int32_t groups;      // 8-channel groups of a row
+  int32_t head_groups; // groups of a head
+  int32_t bits[2];
+  float center[2];
+  uint8_t* stream[2];
+  uint16_t* peak[2];
+  uint8_t* pad;        // a byte between the streams and the maxima, or null
+};
+
+// A wave holds whole token rows, row_lanes lanes each with NV 8-channel groups, so the
+// row maximum is a butterfly inside the wave and each value is read once.  A lane
+// packs its 8 symbols into b bytes; the tile's rows are one stretch of the stream, put
+// together in LDS so that the stream is written in whole 16-byte chunks.  R row steps
+// are loaded before the first is reduced.
+template <int DT, int NV, int R>
+__global__ __launch_bounds__(kQThreads) void cachegen_quantize_kernel(CacheGenQuantParams p) {
+  extern __shared__ __align__(16) uint8_t stage[];
+  const int half = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int RL = p.row_lanes, step_rows = 64 / RL, sub = lane / RL, li = lane & (RL - 1);
+  const uint32_t tile_rows = kQWaves * R * step_rows;
+  const uint32_t t0 = blockIdx.x * tile_rows;
+  const int bits = p.bits[half];
+  const float center = p.center[half];
+
+  int64_t at[NV];  // this lane's groups in a row
+  bool live[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int g = li + v * RL;
+    live[v] = g < p.groups;
+    const int h = g / p.head_groups;
+    at[v] = half * p.s.half + h * p.s.head + static_cast<int64_t>(g - h * p.head_groups) * 8;
+  }
+  Eight<DT> x[R][NV];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t t = t0 + (wave * R + r) * step_rows + sub;
+    const int64_t row = t < p.tokens ? token_offset(p.s, t) : 0;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (t < p.tokens && live[v])
+        x[r][v].load(p.kv, row + at[v]);
+      else
+        x[r][v].clear();
+    }
+  }
+
+  const uint32_t rows = p.tokens - t0 < tile_rows ? p.tokens - t0 : tile_rows;
+  const int64_t row_bytes = static_cast<int64_t>(p.groups) * bits;
+  uint8_t* const dst = p.stream[half] + t0 * row_bytes;
+  const int mis = static_cast<int>(reinterpret_cast<uintptr_t>(dst) & 15);
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const uint32_t local = (wave * R + r) * step_rows + sub;
+    // |x| as an integer: ordered like the value, a NaN above infinity
+    uint32_t top = 0;
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t a = __builtin_bit_cast(uint32_t, x[r][v].get(i)) & 0x7fffffffu;
+        top = top > a ? top : a;
+      }
+    for (int m = 1; m < RL; m <<= 1) {
+      const uint32_t o = __shfl_xor(top, m);
+      top = top > o ? top : o;
+    }
+    const float least = 1e-6f;
+    float peak = __builtin_bit_cast(float, top);
+    if (peak < least) peak = least;
+    const float scale = __fmul_rn(__fdiv_rn(1.0f, peak), center);
+    if (local >= rows) continue;
+    if (li == 0) p.peak[half][t0 + local] = half_bits(peak);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (!live[v]) continue;
+      uint32_t q[2] = {0, 0};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float y = __builtin_rintf(__fadd_rn(__fmul_rn(x[r][v].get(i), scale), center));
+        // a NaN compares false twice and converts to 0
+        if (y < 0.0f) y = 0.0f;
+        if (y > 2.0f * center) y = 2.0f * center;
+        q[i >> 2] |= static_cast<uint32_t>(y == y ? y : 0.0f) << (bits * (i & 3));
+      }
+      const uint64_t packed = q[0] | (static_cast<uint64_t>(q[1]) << (4 * bits));
+      uint8_t* o = stage + mis + local * row_bytes + (li + v * RL) * bits;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < bits) o[i] = static_cast<uint8_t>(packed >> (8 * i));
+    }
+  }
+  __syncthreads();
+  const int total = mis + static_cast<int>(rows * row_bytes);
+  for (int c = threadIdx.x * 16; c < total; c += kQThreads * 16) {
+    uint8_t* const o = dst - mis + c;
+    if (c >= mis && c + 16 <= total) {
+      *reinterpret_cast<u32x4*>(o) = *reinterpret_cast<const u32x4*>(stage + c);
+    } else {  // the tile's ends: the rest of the chunk is another tile's
+      for (int i = 0; i < 16; ++i)
+        if (c + i >= mis && c + i < total) o[i] = stage[c + i];
+    }
+  }
+  if (p.pad && blockIdx.x == 0 && half == 0 && threadIdx.x == 0) *p.pad = 0;
+}
+
+template <int DT, int NV, int R>
+int launch_cachegen(const CacheGenQuantParams& p, hipStream_t stream) {
+  const uint32_t tile_rows = kQWaves * R * (64 / p.row_lanes);
+  const dim3 grid((p.tokens + tile_rows - 1) / tile_rows, 2);
+  const size_t lds = static_cast<size_t>(tile_rows) * p.groups * 8 + 32;
+  hipLaunchKernelGGL((cachegen_quantize_kernel<DT, NV, R>), grid, dim3(kQThreads), lds, stream, p);
+  return check_launch("cachegen_quantize_kernel");
+}
+
+// Groups per lane by row length (at most 4096 channels), and several row steps in
+// flight where the launch still gives every CU two workgroups.
+template <int DT>
+int launch_cachegen_rows(const CacheGenQuantParams& p, hipStream_t stream) {
+  const int64_t steps = (static_cast<int64_t>(p.tokens) * p.row_lanes / 64) * 2 / kQWaves;
+  if (p.groups <= 64)
+    return steps >= 4 * 512 ? launch_cachegen<DT, 1, 4>(p, stream)
+                            : launch_cachegen<DT, 1, 1>(p, stream);
+  if (p.groups <= 128)
+    return steps >= 4 * 512 ? launch_cachegen<DT, 2, 4>(p, stream)
+                            : launch_cachegen<DT, 2, 1>(p, stream);
+  if (p.groups <= 256) return launch_cachegen<DT, 4, 1>(p, stream);
+  return launch_cachegen<DT, 8, 1>(p, stream);
+}
+
+// ---------------------------------------------------------------------------
+// KIVI
+// ---------------------------------------------------------------------------
+
+struct KiviQuantParams {
+  const void* kv;
+  KvStrides s;
+  uint32_t tokens, sink, body;
+  int32_t H, D, C;
+  int32_t group;        // 16, 32, 64 or 128
+  int32_t vgroups;
+  float levels, inv_levels;
+  uint8_t* stream[2];   // packed streams, or one byte per symbol (workspace)
+  uint16_t* scale[2];
+  uint16_t* zero[2];
+  uint16_t* sink_rows[2];
+  uint8_t* pad[8];      // bytes between parts that are written as 0 (null: none)
+  int32_t tiles[2];     // workgroups of the keys, then the values, then the sink rows
+  int32_t chan_tiles[2];
+};
+
+constexpr int kQTokens = 16;  // tokens of a lane
+
+// Minimum and maximum of float16 values, NaN if one is NaN: both as float16 bits in
+// one register for the butterflies.
+struct Range {
+  float lo, hi;
+  __device__ __forceinline__ void start() {
+    lo = __builtin_inff();
+    hi = -__builtin_inff();
+  }
+  __device__ __forceinline__ void add(float x) {
+    lo = (x < lo || x != x) ? x : lo;
+    hi = (x > hi || x != x) ? x : hi;
+  }
+  __device__ __forceinline__ void merge_lane(int mask) {
+    const uint32_t mine = half_bits(lo) | (static_cast<uint32_t>(half_bits(hi)) << 16);
+    const uint32_t o = __shfl_xor(mine, mask);
+    add_lo(static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(o))));
+    add_hi(static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(o >> 16))));
+  }
+  __device__ __forceinline__ void add_lo(float x) { lo = (x < lo || x != x) ? x : lo; }
+  __device__ __forceinline__ void add_hi(float x) { hi = (x > hi || x != x) ? x : hi; }
+};
+
+__device__ __forceinline__ float kivi_scale(const Range& r, float inv_levels) {
+  const float tiny = 1.17549435e-38f;  // the least normal binary32
+  const float s = __fmul_rn(__fsub_rn(r.hi, r.lo), inv_levels);
+  return s < tiny ? tiny : s;
+}
+
+// round(x / scale) clamped to the levels, x / scale the correctly rounded quotient.
+// Its product with the reciprocal is within 2^-21 of it, relatively, so the quotient
+// itself is only evaluated where that could move the rounding (or is not finite).
+__device__ __forceinline__ uint32_t kivi_symbol(float x, float scale, float inv_scale,
+                                                float levels) {
+  float t = __fmul_rn(x, inv_scale);
+  const float near = __builtin_fabsf(__builtin_fabsf(t - __builtin_rintf(t)) - 0.5f);
+  if (!(near > 2.0f * 256.0f / 2097152.0f)) t = __fdiv_rn(x, scale);
+  float y = __builtin_rintf(t);
+  if (y < 0.0f) y = 0.0f;
+  if (y > levels) y = levels;
+  return static_cast<uint32_t>(y == y ? y : 0.0f);
+}
+
+// Writes a lane's run of one plane: 16 symbols (nv of them valid) of SB bits.  SB = 0:
+// one byte per symbol at any address (the packer follows).
+template <int SB>
+__device__ __forceinline__ void store_run(uint8_t* stream, int64_t symbol, const uint32_t (&s)[4],
+                                          int nv) {
+  // s: 16 symbols, one per byte
+  if constexpr (SB == 0) {
+    uint8_t* const o = stream + symbol;
+    if (nv == kQTokens) {
+      *reinterpret_cast<u32x4u*>(o) = u32x4u{s[0], s[1], s[2], s[3]};
+    } else {
+      for (int j = 0; j < nv; ++j)
+        o[j] = static_cast<uint8_t>((j < 8 ? (j < 4 ? s[0] : s[1]) : (j < 12 ? s[2] : s[3])) >>
+                                    (8 * (j & 3)));
+    }
+  } else if constexpr (SB == 8) {
+    *reinterpret_cast<u32x4*>(stream + symbol) = u32x4{s[0], s[1], s[2], s[3]};
+  } else if constexpr (SB == 4) {
+    uint32_t d[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      uint32_t a = s[2 * i] | (s[2 * i] >> 4), b = s[2 * i + 1] | (s[2 * i + 1] >> 4);
+      a = (a & 0xffu) | ((a >> 8) & 0xff00u);
+      b = (b & 0xffu) | ((b >> 8) & 0xff00u);
+      d[i] = a | (b << 16);
+    }
+    *reinterpret_cast<u32x2*>(stream + (symbol >> 1)) = u32x2{d[0], d[1]};
+  } else {
+    uint32_t d = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t a = s[i] | (s[i] >> 6);
+      d |= ((a & 0xfu) | ((a >> 12) & 0xf0u)) << (8 * i);
+    }
+    *reinterpret_cast<uint32_t*>(stream + (symbol >> 2)) = d;
+  }
+}
+
+// A lane owns 8 channels x 16 tokens: it loads 16 row segments of 16 bytes, takes the
+// group ranges, and holds each plane's run of 16 tokens, which it writes packed.  Key
+// tiles (groups along tokens) are 8 lanes along channels x 8 along tokens per wave,
+// value tiles (groups along channels) 16 x 4; a workgroup's waves go along tokens, so
+// a plane's stretch of 2-bit symbols is a whole 128-byte line of keys (64 bytes of
+// values) written by one workgroup.
+template <int HALF, int DT, int SB>
+__device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uint32_t tile) {
+  constexpr int CL = HALF == 0 ? 8 : 16, TL = 64 / CL;  // lanes along channels, tokens
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t ct = tile % p.chan_tiles[HALF], tt = tile / p.chan_tiles[HALF];
+  const int c0 = (ct * CL + (lane & (CL - 1))) * 8;
+  const uint32_t bt0 = ((tt * kQWaves + wave) * TL + lane / CL) * kQTokens;
+  const bool chan_ok = c0 < p.C;
+  const int nv = !chan_ok || bt0 >= p.body
+                     ? 0
+                     : (p.body - bt0 < kQTokens ? static_cast<int>(p.body - bt0) : kQTokens);
+  const int h = c0 / p.D, d0 = c0 - h * p.D;
+  const int64_t col = HALF * p.s.half + h * p.s.head + d0;
+
+  Eight<DT> x[kQTokens];
+#pragma unroll
+  for (int j = 0; j < kQTokens; ++j) {
+    if (j < nv)
+      x[j].load(p.kv, token_offset(p.s, p.sink + bt0 + j) + col);
+    else
+      x[j].clear();
+  }
+  // through float16, as the adapter's canonical tensor
+  auto value = [&](int j, int i) {
+    if constexpr (DT == ORIGAMI_DTYPE_FLOAT16) return x[j].get(i);
+    return static_cast<float>(__builtin_bit_cast(_Float16, half_bits(x[j].get(i))));
+  };
+
+  uint32_t sym[8][4] = {};
+  if constexpr (HALF == 0) {
+    const int lanes = p.group / kQTokens;  // token lanes of a group
+    const uint32_t g = bt0 / p.group;
+    const bool lead = nv > 0 && bt0 % p.group == 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      Range r;
+      r.start();
+#pragma unroll
+      for (int j = 0; j < kQTokens; ++j)
+        if (j < nv) r.add(value(j, i));
+      for (int m = 1; m < lanes; m <<= 1) r.merge_lane(m * CL);
+      const float scale = kivi_scale(r, p.inv_levels);
+      const float inv = __fdiv_rn(1.0f, scale);
+      if (lead) {
+        p.scale[0][static_cast<int64_t>(g) * p.C + c0 + i] = half_bits(scale);
+        p.zero[0][static_cast<int64_t>(g) * p.C + c0 + i] = half_bits(r.lo);
+      }
+#pragma unroll
+      for (int j = 0; j < kQTokens; ++j)
+        sym[i][j >> 2] |= kivi_symbol(__fsub_rn(value(j, i), r.lo), scale, inv, p.levels)
+                          << (8 * (j & 3));
+    }
+  } else {
+    const int lanes = p.group / 8;  // channel lanes of a group
+    const int g = c0 / p.group;
+    const bool lead = chan_ok && c0 % p.group == 0;
+#pragma unroll
+    for (int j = 0; j < kQTokens; ++j) {
+      Range r;
+      r.start();
+      if (chan_ok) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r.add(value(j, i));
+      }
+      for (int m = 1; m < lanes; m <<= 1) r.merge_lane(m);
+      const float scale = kivi_scale(r, p.inv_levels);
+      const float inv = __fdiv_rn(1.0f, scale);
+      if (lead && j < nv) {
+        const int64_t m = static_cast<int64_t>(bt0 + j) * p.vgroups + g;
+        p.scale[1][m] = half_bits(scale);
+        p.zero[1][m] = half_bits(r.lo);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        sym[i][j >> 2] |= kivi_symbol(__fsub_rn(value(j, i), r.lo), scale, inv, p.levels)
+                          << (8 * (j & 3));
+    }
+  }
+  if (nv == 0) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int64_t plane = HALF == 0 ? static_cast<int64_t>(d0 + i) * p.H + h : c0 + i;
+    store_run<SB>(p.stream[HALF], plane * p.body + bt0, sym[i], nv);
+  }
+}
+
+template <int DT, int SB>
+__global__ __launch_bounds__(kQThreads) void kivi_quantize_kernel(KiviQuantParams p) {
+  uint32_t tile = blockIdx.x;
+  if (tile < static_cast<uint32_t>(p.tiles[0])) {
+    kivi_quantize_tile<0, DT, SB>(p, tile);
+    return;
+  }
+  tile -= p.tiles[0];
+  if (tile < static_cast<uint32_t>(p.tiles[1])) {
+    kivi_quantize_tile<1, DT, SB>(p, tile);
+    return;
+  }
+  // sink rows of both halves, 8 channels per thread, and the pad bytes
+  tile -= p.tiles[1];
+  if (tile == 0 && threadIdx.x < 8 && p.pad[threadIdx.x]) *p.pad[threadIdx.x] = 0;
+  const uint32_t G = p.C / 8, n = p.sink * G;
+  const uint32_t i = tile * kQThreads + threadIdx.x;
+  if (i >= 2 * n) return;
+  const int half = i >= n;
+  const uint32_t k = i - half * n, t = k / G, c0 = (k - t * G) * 8;
+  const int h = c0 / p.D, d0 = c0 - h * p.D;
+  Eight<DT> x;
+  x.load(p.kv, half * p.s.half + token_offset(p.s, t) + h * p.s.head + d0);
+  uint16_t* const o = p.sink_rows[half] + static_cast<int64_t>(t) * p.C + c0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) o[j] = half_bits(x.get(j));
+}
+
+template <int DT>
+int launch_kivi(const KiviQuantParams& p, int sb, hipStream_t stream) {
+  const uint32_t sink_tiles = (2 * p.sink * (p.C / 8) + kQThreads - 1) / kQThreads;
+  const dim3 grid(p.tiles[0] + p.tiles[1] + (sink_tiles > 0 ? sink_tiles : 1)), block(kQThreads);
+  switch (sb) {
+    case 0: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 0>), grid, block, 0, stream, p); break;
+    case 2: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 2>), grid, block, 0, stream, p); break;
+    case 4: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 4>), grid, block, 0, stream, p); break;
+    default: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 8>), grid, block, 0, stream, p); break;
+  }
+  return check_launch("kivi_quantize_kernel");
+}
+
+// Checks that both quantizers share; fills `s`.  kv is 16-byte aligned and every row
+// segment of 8 channels with it.
+int check_kv(const void* kv, int64_t dtype, int64_t tokens, int64_t heads, int64_t head_dim,
+             const int64_t* strides, KvStrides* s) {
+  ORIGAMI_REQUIRE(dtype == ORIGAMI_DTYPE_FLOAT16 || dtype == ORIGAMI_DTYPE_BFLOAT16 ||
+                      dtype == ORIGAMI_DTYPE_FLOAT32,
+                  "K/V must be float16, bfloat16 or float32");
+  ORIGAMI_REQUIRE(tokens > 0 && heads > 0 && head_dim > 0,
+                  "tokens, heads, and head_dim must be positive");
+  for (int i = 0; i < 4; ++i)
+    ORIGAMI_REQUIRE(strides[i] >= 0, "K/V strides must be non-negative");
+  ORIGAMI_REQUIRE(strides[4] > 0, "K/V block size must be positive");
+  if (!aligned16(kv) || head_dim % 8 != 0 || strides[0] % 8 != 0 || strides[1] % 8 != 0 ||
+      strides[2] % 8 != 0 || strides[3] % 8 != 0 || tokens > (int64_t(1) << 30) ||
+      heads * head_dim > (int64_t(1) << 24) || strides[4] > UINT32_MAX)
+    return fail(ORIGAMI_ERR_UNSUPPORTED, "the fused quantizers need 16-byte channel groups");
+  *s = KvStrides{strides[0], strides[1], strides[2], strides[3],
+                 static_cast<uint32_t>(strides[4])};
+  return ORIGAMI_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int origami_cachegen_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t heads,
+                              int64_t head_dim, const int64_t* strides, int64_t key_bits,
+                              int64_t value_bits, int64_t key_bins, int64_t value_bins,
+                              uint8_t* payload, int64_t payload_bytes, int64_t value_offset,
+                              int64_t key_max_offset, int64_t value_max_offset,
+                              origami_stream_t stream_) {
+  CacheGenQuantParams p{};
+  if (int rc = check_kv(kv, dtype, tokens, heads, head_dim, strides, &p.s)) return rc;
+  const int64_t C = heads * head_dim;
+  const int64_t bits[2] = {key_bits, value_bits}, bins[2] = {key_bins, value_bins};
+  const int64_t streams[2] = {0, value_offset}, maxima[2] = {key_max_offset, value_max_offset};
+  for (int i = 0; i < 2; ++i) {
+    ORIGAMI_REQUIRE(bits[i] >= 1 && bits[i] <= 8,
+                    "Origami CUDA bitpack supports only 1..8 bit symbols");
+    ORIGAMI_REQUIRE(bins[i] > 3 && bins[i] - 2 < (int64_t(1) << bits[i]),
+                    "CacheGen bins do not fit the symbol width");
+  }
+  if (C > 4096) return fail(ORIGAMI_ERR_UNSUPPORTED, "CacheGen rows of at most 4096 channels");
+  const int64_t bytes[2] = {tokens * C / 8 * key_bits, tokens * C / 8 * value_bits};
+  ORIGAMI_REQUIRE(value_offset >= bytes[0] && key_max_offset >= value_offset + bytes[1] &&
+                      value_max_offset >= key_max_offset + 2 * tokens &&
+                      value_max_offset + 2 * tokens <= payload_bytes,
+                  "CacheGen payload parts overlap or exceed the payload");
+  ORIGAMI_REQUIRE((reinterpret_cast<uintptr_t>(payload) + key_max_offset) % 2 == 0 &&
+                      (reinterpret_cast<uintptr_t>(payload) + value_max_offset) % 2 == 0,
+                  "CacheGen maxima must be at even addresses");
+  p.kv = kv;
+  p.tokens = static_cast<uint32_t>(tokens);
+  p.groups = static_cast<int32_t>(C / 8);
+  p.head_groups = static_cast<int32_t>(head_dim / 8);
+  p.row_lanes = 1;
+  while (p.row_lanes < 64 && p.row_lanes < p.groups) p.row_lanes *= 2;
+  for (int i = 0; i < 2; ++i) {
+    p.bits[i] = static_cast<int32_t>(bits[i]);
+    p.center[i] = static_cast<float>(bins[i] / 2 - 1);
+    p.stream[i] = payload + streams[i];
+    p.peak[i] = reinterpret_cast<uint16_t*>(payload + maxima[i]);
+  }
+  ORIGAMI_REQUIRE(key_max_offset - value_offset - bytes[1] <= 1,
+                  "CacheGen payload has at most one pad byte");
+  if (key_max_offset > value_offset + bytes[1]) p.pad = payload + key_max_offset - 1;
+  const hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+  if (dtype == ORIGAMI_DTYPE_FLOAT32)
+    return launch_cachegen_rows<ORIGAMI_DTYPE_FLOAT32>(p, stream);
+  if (dtype == ORIGAMI_DTYPE_BFLOAT16)
+    return launch_cachegen_rows<ORIGAMI_DTYPE_BFLOAT16>(p, stream);
+  return launch_cachegen_rows<ORIGAMI_DTYPE_FLOAT16>(p, stream);
+}
+
+int origami_kivi_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t heads,
+                          int64_t head_dim, const int64_t* strides, int64_t bits,
+                          int64_t group_size, int64_t sink_tokens, uint8_t* payload,
+                          int64_t payload_bytes, const int64_t* offsets, uint8_t* workspace,
+                          int64_t workspace_bytes, origami_stream_t stream_) {
+  KiviQuantParams p{};
+  if (int rc = check_kv(kv, dtype, tokens, heads, head_dim, strides, &p.s)) return rc;
+  ORIGAMI_REQUIRE(bits == 2 || bits == 3 || bits == 4 || bits == 8,
+                  "KIVI packs 2, 3, 4 or 8 bits");
+  ORIGAMI_REQUIRE(group_size > 0 && sink_tokens >= 0 && sink_tokens < tokens,
+                  "KIVI needs a positive group and a body token");
+  const int64_t C = heads * head_dim, body = tokens - sink_tokens;
+  if (group_size != 16 && group_size != 32 && group_size != 64 && group_size != 128)
+    return fail(ORIGAMI_ERR_UNSUPPORTED, "fused KIVI groups are 16, 32, 64 or 128");
+  const int sb = bits == 3 ? 4 : static_cast<int>(bits);
+  const int64_t key_groups = (body + group_size - 1) / group_size;
+  const int64_t value_groups = (C + group_size - 1) / group_size;
+  const int64_t part[8] = {(C * body * sb + 7) / 8,     (C * body * sb + 7) / 8,
+                           2 * key_groups * C,           2 * key_groups * C,
+                           2 * body * value_groups,      2 * body * value_groups,
+                           2 * sink_tokens * C,          2 * sink_tokens * C};
+  int64_t end = 0;
+  for (int i = 0; i < 8; ++i) {
+    ORIGAMI_REQUIRE(offsets[i] >= end && offsets[i] - end <= 1,
+                    "KIVI payload parts overlap or leave more than a pad byte");
+    if (offsets[i] > end) p.pad[i] = payload + end;
+    ORIGAMI_REQUIRE(i < 2 || (reinterpret_cast<uintptr_t>(payload) + offsets[i]) % 2 == 0,
+                    "KIVI metadata must be at even addresses");
+    end = offsets[i] + part[i];
+  }
+  ORIGAMI_REQUIRE(end <= payload_bytes, "KIVI payload is too small");
+
+  // A lane's run of 16 symbols is whole aligned words of the stream when the planes are
+  // whole runs; otherwise symbols go through the workspace, one per byte, and each
+  // stream is packed from there (2 more bytes of traffic per symbol, but planes may start at any
+  // bit).
+  const bool direct = body % kQTokens == 0 && aligned16(payload) && offsets[1] % 16 == 0;
+  SymbolRun runs[2];
+  if (!direct) {
+    ORIGAMI_REQUIRE(workspace != nullptr && workspace_bytes >= 2 * C * body,
+                    "KIVI workspace is too small");
+    for (int i = 0; i < 2; ++i) {
+      runs[i] = SymbolRun{i * C * body, offsets[i], C * body};
+      if (!pack_runs_aligned(workspace, payload, &runs[i], 1))
+        return fail(ORIGAMI_ERR_UNSUPPORTED, "fused KIVI streams must start on dwords");
+    }
+  }
+  p.kv = kv;
+  p.tokens = static_cast<uint32_t>(tokens);
+  p.sink = static_cast<uint32_t>(sink_tokens);
+  p.body = static_cast<uint32_t>(body);
+  p.H = static_cast<int32_t>(heads);
+  p.D = static_cast<int32_t>(head_dim);
+  p.C = static_cast<int32_t>(C);
+  p.group = static_cast<int32_t>(group_size);
+  p.vgroups = static_cast<int32_t>(value_groups);
+  p.levels = static_cast<float>((1 << bits) - 1);
+  p.inv_levels = 1.0f / p.levels;
+  int64_t grid = 0;
+  for (int i = 0; i < 2; ++i) {
+    p.stream[i] = direct ? payload + offsets[i] : workspace + i * C * body;
+    p.scale[i] = reinterpret_cast<uint16_t*>(payload + offsets[2 + 2 * i]);
+    p.zero[i] = reinterpret_cast<uint16_t*>(payload + offsets[3 + 2 * i]);
+    p.sink_rows[i] = reinterpret_cast<uint16_t*>(payload + offsets[6 + i]);
+    const int64_t chan_lanes = i == 0 ? 8 : 16, tile_tokens = kQWaves * kQTokens * 64 / chan_lanes;
+    p.chan_tiles[i] = static_cast<int32_t>((C + 8 * chan_lanes - 1) / (8 * chan_lanes));
+    const int64_t tiles = p.chan_tiles[i] * ((body + tile_tokens - 1) / tile_tokens);
+    grid += tiles;
+    p.tiles[i] = static_cast<int32_t>(tiles);
+  }
+  if (grid + 2 * sink_tokens * C / 8 / kQThreads + 2 > INT32_MAX ||
+      2 * sink_tokens * (C / 8) > INT32_MAX)
+    return fail(ORIGAMI_ERR_UNSUPPORTED, "KIVI layer exceeds the launch grid");
+  const hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
+  const int store = direct ? sb : 0;
+  int rc = ORIGAMI_OK;
+  if (dtype == ORIGAMI_DTYPE_FLOAT32)
+    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT32>(p, store, stream);
+  else if (dtype == ORIGAMI_DTYPE_BFLOAT16)
+    rc = launch_kivi<ORIGAMI_DTYPE_BFLOAT16>(p, store, stream);
+  else
+    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT16>(p, store, stream);
+  for (int i = 0; i < 2 && !direct && rc == ORIGAMI_OK; ++i)
+    rc = launch_pack_runs(workspace, &runs[i], 1, sb, payload, stream);
+  return rc;
+}
+
+}  // extern "C"

@@ -656,6 +656,63 @@ def kivi_dequantize_to_kv_cache(
 
 
 # ---------------------------------------------------------------------------
+# Fused quantized saves (CacheGen, KIVI)
+# ---------------------------------------------------------------------------
+
+def _quantize_call(name: str, kv: torch.Tensor, dims: Sequence[int], strides: Sequence[int],
+                   *args) -> bool:
+    """Calls a fused quantizer; False where it does not serve these arguments."""
+    strides_arr = _native.i64_array(strides)
+    try:
+        with _device_guard(kv.device):
+            _native.call(name, kv.data_ptr(), _DTYPE_CODES[kv.dtype], *dims,
+                         strides_arr.ctypes.data, *args, _stream_handle(kv.device))
+    except _native.OrigamiNativeError as e:
+        if e.code == _native.ORIGAMI_ERR_UNSUPPORTED:
+            return False
+        raise
+    return True
+
+
+def can_quantize(kv: torch.Tensor) -> bool:
+    """Whether `kv` is a tensor the fused quantizers read (their C entry points
+    check the rest and return False where they do not apply)."""
+    return kv.is_cuda and kv.dtype in _DTYPE_CODES and kv.is_contiguous() and kv.numel() > 0
+
+
+def cachegen_quantize(kv: torch.Tensor, *, dims: Sequence[int], strides: Sequence[int],
+                      key_bits: int, value_bits: int, key_bins: int, value_bins: int,
+                      payload: torch.Tensor, value_offset: int, key_max_offset: int,
+                      value_max_offset: int) -> bool:
+    """One layer's CacheGen payload from its K/V in one pass
+    (cachegen_adapter.py:246-340 of the reference): dims (tokens, heads,
+    head_dim), strides (half, block, token, head, tokens per block) of `kv`
+    in elements.  False, with nothing done, where the kernel does not apply."""
+    return _quantize_call("origami_cachegen_quantize", kv, dims, strides, int(key_bits),
+                          int(value_bits), int(key_bins), int(value_bins), payload.data_ptr(),
+                          payload.numel(), int(value_offset), int(key_max_offset),
+                          int(value_max_offset))
+
+
+def kivi_quantize(kv: torch.Tensor, *, dims: Sequence[int], strides: Sequence[int], bits: int,
+                  group_size: int, sink_tokens: int, payload: torch.Tensor,
+                  offsets: Sequence[int]) -> bool:
+    """One layer's KIVI payload from its K/V (kivi_adapter.py:229-450 of the
+    reference), parts at `offsets` of `payload`; dims, strides and the result
+    as cachegen_quantize."""
+    tokens, heads, head_dim = dims
+    body = tokens - sink_tokens
+    work = None
+    if body % 16 or int(offsets[1]) % 16:
+        work = torch.empty((2 * body * heads * head_dim,), dtype=torch.uint8, device=kv.device)
+    offs = _native.i64_array(offsets)
+    return _quantize_call("origami_kivi_quantize", kv, dims, strides, int(bits), int(group_size),
+                          int(sink_tokens), payload.data_ptr(), payload.numel(),
+                          offs.ctypes.data, work.data_ptr() if work is not None else 0,
+                          work.numel() if work is not None else 0)
+
+
+# ---------------------------------------------------------------------------
 # Reference extension surface (origami_bitpack_cuda_v6, cpp:894-903)
 # ---------------------------------------------------------------------------
 

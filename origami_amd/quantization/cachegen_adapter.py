@@ -16,8 +16,9 @@ onto `bins` levels whose count depends on the layer (cachegen_adapter.py:
   unpack + dequantize + paged scatter (native_gpu.
   cachegen_unpack_dequantize_to_kv_cache) in one pass.
 
-Quantize and the unfused dequantize use the reference's torch expressions
-(float32 tensor ops, round half to even); they run on whatever device the
+Quantize runs as one HIP kernel on GPU tensors (native_gpu.cachegen_quantize), with the
+rounding of the reference's torch expressions (float32 tensor ops, round half to even),
+which are used elsewhere and by the unfused dequantize; those run on whatever device the
 input is on.  Bit packing and unpacking run on the GPU (liborigami_layout.so).
 """
 from __future__ import annotations
@@ -124,6 +125,34 @@ def canonicalize(kv: torch.Tensor) -> tuple[torch.Tensor, str]:
         return t.permute(1, 0, 2, 3).contiguous(), "tokens_kv_heads_dim"
     raise ValueError("expected a KV cache layer with a key/value axis; "
                      f"got shape {tuple(kv.shape)}")
+
+
+def kv_geometry(t: torch.Tensor) -> tuple[str, tuple[int, int, int], tuple[int, ...]]:
+    """canonicalize without the copy: layout name, (tokens, heads, head_dim) and the
+    element strides (half, block, token, head, tokens per block) of a contiguous K/V
+    tensor, for the fused quantizers."""
+    s = [int(x) for x in t.shape]
+    if t.dim() == 5 and s[0] == 2:
+        T, (H, D) = s[1] * s[2], s[3:]
+        return "kv_blocks_block_heads_dim", (T, H, D), (T * H * D, 0, H * D, D, T)
+    if t.dim() == 5 and s[1] == 2:
+        bs, H, D = s[2:]
+        row = H * D
+        return "blocks_kv_block_heads_dim", (s[0] * bs, H, D), (bs * row, 2 * bs * row, row, D, bs)
+    if t.dim() == 5 and s[2] == 2:
+        T, (H, D) = s[0] * s[1], s[3:]
+        return "blocks_block_kv_heads_dim", (T, H, D), (H * D, 0, 2 * H * D, D, T)
+    if t.dim() == 4 and s[0] == 2:
+        if s[1] <= 128 and s[2] > s[1]:
+            H, T, D = s[1:]
+            return "kv_heads_tokens_dim", (T, H, D), (H * T * D, 0, D, T * D, T)
+        T, H, D = s[1:]
+        return "kv_tokens_heads_dim", (T, H, D), (T * H * D, 0, H * D, D, T)
+    if t.dim() == 4 and s[1] == 2:
+        T, _, H, D = s
+        return "tokens_kv_heads_dim", (T, H, D), (H * D, 0, 2 * H * D, D, T)
+    raise ValueError("expected a KV cache layer with a key/value axis; "
+                     f"got shape {tuple(t.shape)}")
 
 
 def restore_layout(canonical: torch.Tensor, metadata: dict[str, Any]) -> torch.Tensor:
@@ -249,16 +278,44 @@ class CacheGenAdapter(QuantizerAdapter):
         q = torch.round(x * (center / max_abs) + center).clamp(0, center * 2).to(torch.uint8)
         return q, max_abs.to(torch.float16)
 
+    def _payload(self, tensor: torch.Tensor, kbins: int, vbins: int, kbits: int,
+                 vbits: int) -> torch.Tensor:
+        """The payload by tensor operations, on the tensor's device."""
+        canonical, _ = canonicalize(tensor)
+        key_q, key_max = self.quantize_plane(canonical[0], kbins)
+        value_q, value_max = self.quantize_plane(canonical[1], vbins)
+        if self.bitpacked:
+            parts = [pack_linear(key_q, kbits), pack_linear(value_q, vbits)]
+        else:
+            parts = [key_q.reshape(-1), value_q.reshape(-1)]
+        dev = parts[0].device
+        if sum(int(p.numel()) for p in parts) % 2:
+            parts.append(torch.zeros((1,), dtype=torch.uint8, device=dev))
+        parts += [fp16_bytes(key_max).to(dev), fp16_bytes(value_max).to(dev)]
+        return torch.cat(parts).contiguous()
+
+    def _fused_payload(self, tensor: torch.Tensor, dims, strides, widths, bins, offsets,
+                       size: int) -> torch.Tensor | None:
+        """The same bytes in one pass over a GPU tensor (origami_cachegen_quantize),
+        or None where that kernel does not apply."""
+        if not native_gpu.can_quantize(tensor):
+            return None
+        symbols = torch.empty((size,), dtype=torch.uint8, device=tensor.device)
+        done = native_gpu.cachegen_quantize(
+            tensor, dims=dims, strides=strides, key_bits=widths[0], value_bits=widths[1],
+            key_bins=bins[0], value_bins=bins[1], payload=symbols, value_offset=offsets[1],
+            key_max_offset=offsets[2], value_max_offset=offsets[3])
+        return symbols if done else None
+
     def quantize(self, kv: torch.Tensor, *, request: Any | None = None,
                  layer_group: Any | None = None, stream: Any | None = None) -> QuantizedKV:
         del request, stream
-        canonical, layout = canonicalize(kv)
+        tensor = kv.detach().contiguous()
+        layout, (tokens, heads, head_dim), strides = kv_geometry(tensor)
         layer = layer_index(layer_group)
         kbins, vbins = self.key_bins(layer), self.value_bins(layer)
         kbits, vbits = bits_for_bins(kbins), bits_for_bins(vbins)
-        key_q, key_max = self.quantize_plane(canonical[0], kbins)
-        value_q, value_max = self.quantize_plane(canonical[1], vbins)
-        tokens, heads, head_dim = (int(x) for x in canonical.shape[1:])
+        count = tokens * heads * head_dim
         meta: dict[str, Any] = {
             "format": BITPACKED if self.bitpacked else STRUCTURED,
             "version": 2,
@@ -276,30 +333,27 @@ class CacheGenAdapter(QuantizerAdapter):
             "num_heads": heads,
             "head_dim": head_dim,
             "channel_count": heads * head_dim,
-            "key_q_numel": int(key_q.numel()),
-            "value_q_numel": int(value_q.numel()),
-            "key_max_numel": int(key_max.numel()),
-            "value_max_numel": int(value_max.numel()),
+            "key_q_numel": count,
+            "value_q_numel": count,
+            "key_max_numel": tokens,
+            "value_max_numel": tokens,
         }
-        if self.bitpacked:
-            streams = [pack_linear(key_q, kbits), pack_linear(value_q, vbits)]
-            names = ["key_stream", "value_stream"]
-        else:
-            streams = [key_q.reshape(-1), value_q.reshape(-1)]
-            names = ["key_q", "value_q"]
-        parts, cursor = [], 0
-        dev = streams[0].device
-        for name, part in zip(names + ["key_max", "value_max"],
-                              streams + [fp16_bytes(key_max).to(dev), fp16_bytes(value_max).to(dev)]):
-            if name.endswith("_max") and cursor % 2:     # float16 views need even offsets
-                parts.append(torch.zeros((1,), dtype=torch.uint8, device=dev))
-                cursor += 1
+        names = ["key_stream", "value_stream"] if self.bitpacked else ["key_q", "value_q"]
+        widths = [kbits, vbits] if self.bitpacked else [8, 8]
+        sizes = [(count * w + 7) // 8 for w in widths] + [2 * tokens, 2 * tokens]
+        offsets, cursor = [], 0
+        for name, size in zip(names + ["key_max", "value_max"], sizes):
+            if name.endswith("_max"):
+                cursor += cursor % 2                     # float16 views need even offsets
             meta[f"{name}_offset"] = cursor
             if name.endswith("_stream"):
-                meta[f"{name}_bytes"] = int(part.numel())
-            parts.append(part.reshape(-1).to(torch.uint8))
-            cursor += int(part.numel())
-        symbols = torch.cat(parts).contiguous()
+                meta[f"{name}_bytes"] = size
+            offsets.append(cursor)
+            cursor += size
+        symbols = self._fused_payload(tensor, (tokens, heads, head_dim), strides, widths,
+                                      (kbins, vbins), offsets, cursor)
+        if symbols is None:
+            symbols = self._payload(tensor, kbins, vbins, kbits, vbits)
         meta.update({
             "symbol_byte_count": int(symbols.numel()),
             "origami_bits": 8,

@@ -33,6 +33,7 @@ from origami_amd.quantization.cachegen_adapter import (
     dtype_from_metadata,
     fp16_bytes,
     fp16_view,
+    kv_geometry,
     restore_layout,
 )
 
@@ -163,13 +164,11 @@ class KiviAdapter(QuantizerAdapter):
         return (q.to(torch.uint8).reshape(rows, groups * group)[:, :cols].contiguous(),
                 scale.to(torch.float16).contiguous(), zero.to(torch.float16).contiguous())
 
-    def quantize(self, kv: torch.Tensor, *, request: Any | None = None,
-                 layer_group: Any | None = None, stream: Any | None = None) -> QuantizedKV:
-        del request, layer_group, stream
-        canonical, layout = canonicalize(kv)
+    def _payload(self, tensor: torch.Tensor, sink: int) -> torch.Tensor:
+        """The payload by tensor operations, on the tensor's device."""
+        canonical, _ = canonicalize(tensor)
         c16 = canonical.to(torch.float16).contiguous()
         tokens, heads, head_dim = (int(x) for x in c16.shape[1:])
-        sink = min(self.sink_tokens, tokens)
         body = tokens - sink
         cols = heads * head_dim
         key_q, key_scale, key_zero = self.quantize_key_per_channel(
@@ -179,23 +178,53 @@ class KiviAdapter(QuantizerAdapter):
         data_shape = (1, body, heads, head_dim)
         key_stream = pack_ordered(key_q.reshape(data_shape), KEY_ORDER, self.bits)
         value_stream = pack_ordered(value_q.reshape(data_shape), VALUE_ORDER, self.bits)
-        parts, offsets, cursor = [], {}, 0
+        parts, cursor = [], 0
         dev = key_stream.device
-        named = [("key_stream", key_stream, 1), ("value_stream", value_stream, 1),
-                 ("key_scale", fp16_bytes(key_scale), 2), ("key_zero", fp16_bytes(key_zero), 2),
-                 ("value_scale", fp16_bytes(value_scale), 2),
-                 ("value_zero", fp16_bytes(value_zero), 2),
-                 ("key_sink", fp16_bytes(c16[0, :sink]), 2),
-                 ("value_sink", fp16_bytes(c16[1, :sink]), 2)]
-        for name, data, align in named:
+        named = [(key_stream, 1), (value_stream, 1), (fp16_bytes(key_scale), 2),
+                 (fp16_bytes(key_zero), 2), (fp16_bytes(value_scale), 2),
+                 (fp16_bytes(value_zero), 2), (fp16_bytes(c16[0, :sink]), 2),
+                 (fp16_bytes(c16[1, :sink]), 2)]
+        for data, align in named:
             pad = (-cursor) % align
             if pad:
                 parts.append(torch.zeros((pad,), dtype=torch.uint8, device=dev))
                 cursor += pad
-            offsets[name] = cursor
             parts.append(data.reshape(-1).to(dev, torch.uint8))
             cursor += int(data.numel())
-        symbols = torch.cat(parts).contiguous()
+        return torch.cat(parts).contiguous()
+
+    def quantize(self, kv: torch.Tensor, *, request: Any | None = None,
+                 layer_group: Any | None = None, stream: Any | None = None) -> QuantizedKV:
+        del request, layer_group, stream
+        tensor = kv.detach().contiguous()
+        layout, (tokens, heads, head_dim), strides = kv_geometry(tensor)
+        sink = min(self.sink_tokens, tokens)
+        body = tokens - sink
+        cols = heads * head_dim
+        key_groups = (body + self.group_size - 1) // self.group_size
+        value_groups = (cols + self.group_size - 1) // self.group_size
+        stored = 4 if self.bits == 3 else self.bits
+        stream_bytes = (body * cols * stored + 7) // 8
+        sizes = {"key_stream": stream_bytes, "value_stream": stream_bytes,
+                 "key_scale": 2 * key_groups * cols, "key_zero": 2 * key_groups * cols,
+                 "value_scale": 2 * body * value_groups, "value_zero": 2 * body * value_groups,
+                 "key_sink": 2 * sink * cols, "value_sink": 2 * sink * cols}
+        offsets, cursor = {}, 0
+        for name, size in sizes.items():
+            if not name.endswith("_stream"):
+                cursor += cursor % 2
+            offsets[name] = cursor
+            cursor += size
+        symbols = None
+        if body > 0 and native_gpu.can_quantize(tensor):
+            symbols = torch.empty((cursor,), dtype=torch.uint8, device=tensor.device)
+            if not native_gpu.kivi_quantize(
+                    tensor, dims=(tokens, heads, head_dim), strides=strides, bits=self.bits,
+                    group_size=self.group_size, sink_tokens=sink, payload=symbols,
+                    offsets=list(offsets.values())):
+                symbols = None
+        if symbols is None:
+            symbols = self._payload(tensor, sink)
         meta: dict[str, Any] = {
             "format": FORMAT,
             "version": 1,
@@ -207,9 +236,9 @@ class KiviAdapter(QuantizerAdapter):
             "num_heads": heads,
             "head_dim": head_dim,
             "channel_count": cols,
-            "key_groups": (body + self.group_size - 1) // self.group_size,
-            "value_groups": (cols + self.group_size - 1) // self.group_size,
-            "data_shape": list(data_shape),
+            "key_groups": key_groups,
+            "value_groups": value_groups,
+            "data_shape": [1, body, heads, head_dim],
             "key_order": list(KEY_ORDER),
             "value_order": list(VALUE_ORDER),
             "dtype": str(kv.dtype).replace("torch.", ""),
@@ -223,12 +252,12 @@ class KiviAdapter(QuantizerAdapter):
         for name, off in offsets.items():
             meta[f"{name}_offset"] = int(off)
         meta.update({
-            "key_stream_bytes": int(key_stream.numel()),
-            "value_stream_bytes": int(value_stream.numel()),
-            "key_scale_numel": int(key_scale.numel()),
-            "key_zero_numel": int(key_zero.numel()),
-            "value_scale_numel": int(value_scale.numel()),
-            "value_zero_numel": int(value_zero.numel()),
+            "key_stream_bytes": stream_bytes,
+            "value_stream_bytes": stream_bytes,
+            "key_scale_numel": key_groups * cols,
+            "key_zero_numel": key_groups * cols,
+            "value_scale_numel": body * value_groups,
+            "value_zero_numel": body * value_groups,
             "key_sink_numel": int(sink * cols),
             "value_sink_numel": int(sink * cols),
         })
