@@ -12,10 +12,12 @@
 //
 // HBM bounds both: 4 bytes read and b / 4 bytes written per (K, V) pair of 16-bit
 // values.  16384 tokens of 8 heads x 128, bf16, with the copy of the payload into its
-// stored chunks: CacheGen 573 -> 30.8 us, KIVI (2 bits) 1032 -> 61.0 us.
+// stored chunks: CacheGen 573 -> 26.7 us, KIVI (2 bits) 1025 -> 33.3 us.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "origami_internal.h"
 #include "origami_layout.h"
@@ -27,6 +29,8 @@ namespace {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4u __attribute__((ext_vector_type(4), aligned(1)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kQThreads = 256;
 constexpr int kQWaves = kQThreads / 64;
@@ -61,10 +65,6 @@ struct Eight {
       w[4 * i + 2] = x.z;
       w[4 * i + 3] = x.w;
     }
-  }
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int i = 0; i < kWords; ++i) w[i] = 0;
   }
   __device__ __forceinline__ float get(int i) const {
     if constexpr (DT == ORIGAMI_DTYPE_FLOAT32) {
@@ -117,12 +117,16 @@ __global__ __launch_bounds__(kQThreads) void cachegen_quantize_kernel(CacheGenQu
   const int bits = p.bits[half];
   const float center = p.center[half];
 
+  // Every lane loads: one past the row's groups takes the last group again and one past
+  // the last token that token, which changes no maximum, so no branch keeps the R * NV
+  // loads from being in flight together (with branches the compiler moved them down to
+  // their uses: the save of 16384 tokens took 30.8 us, 26.7 without).
   int64_t at[NV];  // this lane's groups in a row
   bool live[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int g = li + v * RL;
-    live[v] = g < p.groups;
+    live[v] = li + v * RL < p.groups;
+    const int g = live[v] ? li + v * RL : p.groups - 1;
     const int h = g / p.head_groups;
     at[v] = half * p.s.half + h * p.s.head + static_cast<int64_t>(g - h * p.head_groups) * 8;
   }
@@ -130,15 +134,11 @@ __global__ __launch_bounds__(kQThreads) void cachegen_quantize_kernel(CacheGenQu
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const uint32_t t = t0 + (wave * R + r) * step_rows + sub;
-    const int64_t row = t < p.tokens ? token_offset(p.s, t) : 0;
+    const int64_t row = token_offset(p.s, t < p.tokens ? t : p.tokens - 1);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-      if (t < p.tokens && live[v])
-        x[r][v].load(p.kv, row + at[v]);
-      else
-        x[r][v].clear();
-    }
+    for (int v = 0; v < NV; ++v) x[r][v].load(p.kv, row + at[v]);
   }
+  asm volatile("" ::: "memory");
 
   const uint32_t rows = p.tokens - t0 < tile_rows ? p.tokens - t0 : tile_rows;
   const int64_t row_bytes = static_cast<int64_t>(p.groups) * bits;
@@ -172,11 +172,10 @@ __global__ __launch_bounds__(kQThreads) void cachegen_quantize_kernel(CacheGenQu
       uint32_t q[2] = {0, 0};
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float y = __builtin_rintf(__fadd_rn(__fmul_rn(x[r][v].get(i), scale), center));
-        // a NaN compares false twice and converts to 0
-        if (y < 0.0f) y = 0.0f;
-        if (y > 2.0f * center) y = 2.0f * center;
-        q[i >> 2] |= static_cast<uint32_t>(y == y ? y : 0.0f) << (bits * (i & 3));
+        // |x| <= peak, so the rounded value lies in [0, 2 * center]; the maximum is for
+        // NaNs, which become 0
+        const float y = __builtin_rintf(__fadd_rn(__fmul_rn(x[r][v].get(i), scale), center));
+        q[i >> 2] |= static_cast<uint32_t>(fmaxf(y, 0.0f)) << (bits * (i & 3));
       }
       const uint64_t packed = q[0] | (static_cast<uint64_t>(q[1]) << (4 * bits));
       uint8_t* o = stage + mis + local * row_bytes + (li + v * RL) * bits;
@@ -234,7 +233,7 @@ struct KiviQuantParams {
   int32_t H, D, C;
   int32_t group;        // 16, 32, 64 or 128
   int32_t vgroups;
-  float levels, inv_levels;
+  float inv_levels;
   uint8_t* stream[2];   // packed streams, or one byte per symbol (workspace)
   uint16_t* scale[2];
   uint16_t* zero[2];
@@ -246,93 +245,124 @@ struct KiviQuantParams {
 
 constexpr int kQTokens = 16;  // tokens of a lane
 
-// Minimum and maximum of float16 values, NaN if one is NaN: both as float16 bits in
-// one register for the butterflies.
-struct Range {
-  float lo, hi;
-  __device__ __forceinline__ void start() {
-    lo = __builtin_inff();
-    hi = -__builtin_inff();
-  }
-  __device__ __forceinline__ void add(float x) {
-    lo = (x < lo || x != x) ? x : lo;
-    hi = (x > hi || x != x) ? x : hi;
-  }
-  __device__ __forceinline__ void merge_lane(int mask) {
-    const uint32_t mine = half_bits(lo) | (static_cast<uint32_t>(half_bits(hi)) << 16);
-    const uint32_t o = __shfl_xor(mine, mask);
-    add_lo(static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(o))));
-    add_hi(static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(o >> 16))));
-  }
-  __device__ __forceinline__ void add_lo(float x) { lo = (x < lo || x != x) ? x : lo; }
-  __device__ __forceinline__ void add_hi(float x) { hi = (x > hi || x != x) ? x : hi; }
+// Two float16 values per register: the ranges are taken on pairs.
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_pk_max_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float low_half(uint32_t v) {
+  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(v)));
+}
+__device__ __forceinline__ float high_half(uint32_t v) {
+  return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(v >> 16)));
+}
+
+// One quantization group: zero point (its minimum), scale and the scale's reciprocal.
+struct Group {
+  float zero, scale, inv;
 };
 
-__device__ __forceinline__ float kivi_scale(const Range& r, float inv_levels) {
+// `range` holds the minimum (low) and the negated maximum (high).
+__device__ __forceinline__ Group make_group(uint32_t range, bool nan, float inv_levels) {
   const float tiny = 1.17549435e-38f;  // the least normal binary32
-  const float s = __fmul_rn(__fsub_rn(r.hi, r.lo), inv_levels);
-  return s < tiny ? tiny : s;
+  Group g;
+  g.zero = nan ? __builtin_nanf("") : low_half(range);
+  const float top = nan ? __builtin_nanf("") : high_half(range ^ 0x80000000u);
+  const float s = __fmul_rn(__fsub_rn(top, g.zero), inv_levels);
+  g.scale = s < tiny ? tiny : s;
+  g.inv = __fdiv_rn(1.0f, g.scale);
+  return g;
 }
 
-// round(x / scale) clamped to the levels, x / scale the correctly rounded quotient.
-// Its product with the reciprocal is within 2^-21 of it, relatively, so the quotient
-// itself is only evaluated where that could move the rounding (or is not finite).
-__device__ __forceinline__ uint32_t kivi_symbol(float x, float scale, float inv_scale,
-                                                float levels) {
-  float t = __fmul_rn(x, inv_scale);
-  const float near = __builtin_fabsf(__builtin_fabsf(t - __builtin_rintf(t)) - 0.5f);
-  if (!(near > 2.0f * 256.0f / 2097152.0f)) t = __fdiv_rn(x, scale);
-  float y = __builtin_rintf(t);
-  if (y < 0.0f) y = 0.0f;
-  if (y > levels) y = levels;
-  return static_cast<uint32_t>(y == y ? y : 0.0f);
+// round((x - zero) / scale) in [0, levels], with the correctly rounded quotient: the
+// product with the correctly rounded reciprocal, corrected twice by its remainder
+// (Markstein's division; nothing underflows here, as a scale is the least normal number
+// where the group has one value, and at least 2^-32 elsewhere).  An infinite or NaN
+// scale gives a NaN, whose symbol is 0 like that of the quotient.
+__device__ __forceinline__ float kivi_symbol(float x, const Group& g) {
+  const float d = __fsub_rn(x, g.zero);
+  const float q0 = __fmul_rn(d, g.inv);
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, g.scale, d), g.inv, q0);
+  const float q2 = __builtin_fmaf(__builtin_fmaf(-q1, g.scale, d), g.inv, q1);
+  return __builtin_rintf(fmaxf(q2, 0.0f));
 }
 
-// Writes a lane's run of one plane: 16 symbols (nv of them valid) of SB bits.  SB = 0:
-// one byte per symbol at any address (the packer follows).
-template <int SB>
-__device__ __forceinline__ void store_run(uint8_t* stream, int64_t symbol, const uint32_t (&s)[4],
+// A lane's run of one plane: 16 symbols of W bits, gathered as exact binary32 sums of
+// 16 / W symbols each.
+template <int W>
+struct PlaneRun {
+  static constexpr int kPer = 16 / W;         // symbols of a sum
+  static constexpr int kSums = 16 / kPer;
+  float sum[kSums];
+
+  template <int J>
+  __device__ __forceinline__ void put(float symbol) {
+    constexpr float weight = static_cast<float>(1u << (W * (J % kPer)));
+    if constexpr (J % kPer == 0)
+      sum[J / kPer] = symbol;
+    else
+      sum[J / kPer] = __builtin_fmaf(symbol, weight, sum[J / kPer]);
+  }
+  __device__ __forceinline__ uint32_t word(int i) const {
+    return static_cast<uint32_t>(sum[2 * i]) | (static_cast<uint32_t>(sum[2 * i + 1]) << 16);
+  }
+};
+
+// Writes a run at symbol `symbol` of its stream.  BYTES: W = 8 at any address, `nv`
+// symbols (the packer follows); else a whole run on an aligned word.
+template <int W, bool BYTES>
+__device__ __forceinline__ void store_run(uint8_t* stream, int64_t symbol, const PlaneRun<W>& r,
                                           int nv) {
-  // s: 16 symbols, one per byte
-  if constexpr (SB == 0) {
-    uint8_t* const o = stream + symbol;
+  uint8_t* const o = stream + (symbol * W >> 3);
+  if constexpr (BYTES) {
+    const uint32_t w[4] = {r.word(0), r.word(1), r.word(2), r.word(3)};
     if (nv == kQTokens) {
-      *reinterpret_cast<u32x4u*>(o) = u32x4u{s[0], s[1], s[2], s[3]};
+      *reinterpret_cast<u32x4u*>(o) = u32x4u{w[0], w[1], w[2], w[3]};
     } else {
-      for (int j = 0; j < nv; ++j)
-        o[j] = static_cast<uint8_t>((j < 8 ? (j < 4 ? s[0] : s[1]) : (j < 12 ? s[2] : s[3])) >>
-                                    (8 * (j & 3)));
-    }
-  } else if constexpr (SB == 8) {
-    *reinterpret_cast<u32x4*>(stream + symbol) = u32x4{s[0], s[1], s[2], s[3]};
-  } else if constexpr (SB == 4) {
-    uint32_t d[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      uint32_t a = s[2 * i] | (s[2 * i] >> 4), b = s[2 * i + 1] | (s[2 * i + 1] >> 4);
-      a = (a & 0xffu) | ((a >> 8) & 0xff00u);
-      b = (b & 0xffu) | ((b >> 8) & 0xff00u);
-      d[i] = a | (b << 16);
+      for (int j = 0; j < kQTokens; ++j)
+        if (j < nv) o[j] = static_cast<uint8_t>(w[j >> 2] >> (8 * (j & 3)));
     }
-    *reinterpret_cast<u32x2*>(stream + (symbol >> 1)) = u32x2{d[0], d[1]};
+  } else if constexpr (W == 8) {
+    *reinterpret_cast<u32x4*>(o) = u32x4{r.word(0), r.word(1), r.word(2), r.word(3)};
+  } else if constexpr (W == 4) {
+    *reinterpret_cast<u32x2*>(o) = u32x2{r.word(0), r.word(1)};
   } else {
-    uint32_t d = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t a = s[i] | (s[i] >> 6);
-      d |= ((a & 0xfu) | ((a >> 12) & 0xf0u)) << (8 * i);
-    }
-    *reinterpret_cast<uint32_t*>(stream + (symbol >> 2)) = d;
+    *reinterpret_cast<uint32_t*>(o) = r.word(0);
   }
 }
 
-// A lane owns 8 channels x 16 tokens: it loads 16 row segments of 16 bytes, takes the
-// group ranges, and holds each plane's run of 16 tokens, which it writes packed.  Key
-// tiles (groups along tokens) are 8 lanes along channels x 8 along tokens per wave,
-// value tiles (groups along channels) 16 x 4; a workgroup's waves go along tokens, so
-// a plane's stretch of 2-bit symbols is a whole 128-byte line of keys (64 bytes of
-// values) written by one workgroup.
-template <int HALF, int DT, int SB>
+// Calls f(std::integral_constant<int, i>) for i = 0 .. N - 1.
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) {
+  if constexpr (N > 0) {
+    each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+// A lane owns 8 channels x 16 tokens: it loads 16 row segments of 16 bytes, rounds them
+// to float16 pairs, takes the group ranges, and holds each plane's run of 16 tokens,
+// which it writes packed.  Key tiles (groups along tokens) are 8 lanes along channels x
+// 8 along tokens per wave, value tiles (groups along channels) 16 x 4; a workgroup's
+// waves go along tokens, so a plane's stretch of 2-bit symbols is a whole 128-byte line
+// of keys (64 bytes of values) written by one workgroup.  Lanes past the last token or
+// channel load the last one again, which changes no range of a group they share.
+// With the loads in flight the arithmetic bounds it: ranges on pairs, a branch-free
+// division and symbols gathered by fused multiply-adds took the save of 16384 tokens
+// from 61.0 us (scalar ranges, a branch per quotient, shifts) to 33.3.
+template <int HALF, int DT, int W, bool BYTES>
 __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uint32_t tile) {
   constexpr int CL = HALF == 0 ? 8 : 16, TL = 64 / CL;  // lanes along channels, tokens
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -343,91 +373,133 @@ __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uin
   const int nv = !chan_ok || bt0 >= p.body
                      ? 0
                      : (p.body - bt0 < kQTokens ? static_cast<int>(p.body - bt0) : kQTokens);
-  const int h = c0 / p.D, d0 = c0 - h * p.D;
+  const int cl = chan_ok ? c0 : p.C - 8;
+  const int h = cl / p.D, d0 = cl - h * p.D;
   const int64_t col = HALF * p.s.half + h * p.s.head + d0;
 
-  Eight<DT> x[kQTokens];
-#pragma unroll
-  for (int j = 0; j < kQTokens; ++j) {
-    if (j < nv)
-      x[j].load(p.kv, token_offset(p.s, p.sink + bt0 + j) + col);
-    else
-      x[j].clear();
-  }
-  // through float16, as the adapter's canonical tensor
-  auto value = [&](int j, int i) {
-    if constexpr (DT == ORIGAMI_DTYPE_FLOAT16) return x[j].get(i);
-    return static_cast<float>(__builtin_bit_cast(_Float16, half_bits(x[j].get(i))));
-  };
-
-  uint32_t sym[8][4] = {};
-  if constexpr (HALF == 0) {
-    const int lanes = p.group / kQTokens;  // token lanes of a group
-    const uint32_t g = bt0 / p.group;
-    const bool lead = nv > 0 && bt0 % p.group == 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      Range r;
-      r.start();
-#pragma unroll
-      for (int j = 0; j < kQTokens; ++j)
-        if (j < nv) r.add(value(j, i));
-      for (int m = 1; m < lanes; m <<= 1) r.merge_lane(m * CL);
-      const float scale = kivi_scale(r, p.inv_levels);
-      const float inv = __fdiv_rn(1.0f, scale);
-      if (lead) {
-        p.scale[0][static_cast<int64_t>(g) * p.C + c0 + i] = half_bits(scale);
-        p.zero[0][static_cast<int64_t>(g) * p.C + c0 + i] = half_bits(r.lo);
-      }
-#pragma unroll
-      for (int j = 0; j < kQTokens; ++j)
-        sym[i][j >> 2] |= kivi_symbol(__fsub_rn(value(j, i), r.lo), scale, inv, p.levels)
-                          << (8 * (j & 3));
-    }
-  } else {
-    const int lanes = p.group / 8;  // channel lanes of a group
-    const int g = c0 / p.group;
-    const bool lead = chan_ok && c0 % p.group == 0;
+  uint32_t v[kQTokens][4];  // float16 pairs
+  {
+    const uint32_t last = p.tokens - 1;
+    uint32_t t = p.sink + bt0 < last ? p.sink + bt0 : last;
+    uint32_t blk = t / p.s.block_tokens, off = t - blk * p.s.block_tokens;
+    Eight<DT> x[kQTokens];
 #pragma unroll
     for (int j = 0; j < kQTokens; ++j) {
-      Range r;
-      r.start();
-      if (chan_ok) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r.add(value(j, i));
+      x[j].load(p.kv, static_cast<int64_t>(blk) * p.s.block +
+                          static_cast<int64_t>(off) * p.s.token + col);
+      if (t < last) {
+        ++t;
+        if (++off == p.s.block_tokens) {
+          off = 0;
+          ++blk;
+        }
       }
-      for (int m = 1; m < lanes; m <<= 1) r.merge_lane(m);
-      const float scale = kivi_scale(r, p.inv_levels);
-      const float inv = __fdiv_rn(1.0f, scale);
-      if (lead && j < nv) {
-        const int64_t m = static_cast<int64_t>(bt0 + j) * p.vgroups + g;
-        p.scale[1][m] = half_bits(scale);
-        p.zero[1][m] = half_bits(r.lo);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        sym[i][j >> 2] |= kivi_symbol(__fsub_rn(value(j, i), r.lo), scale, inv, p.levels)
-                          << (8 * (j & 3));
     }
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < kQTokens; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if constexpr (DT == ORIGAMI_DTYPE_FLOAT16) {
+          v[j][k] = x[j].w[k];
+        } else {
+          const f32x2 pair = {x[j].get(2 * k), x[j].get(2 * k + 1)};
+          v[j][k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, f16x2));
+        }
+      }
+  }
+
+  PlaneRun<W> run[8];
+  const uint32_t kAbs = 0x7fff7fffu, kNegHigh = 0x80000000u;
+  if constexpr (HALF == 0) {
+    const int lanes = p.group / kQTokens;  // token lanes of a group
+    uint32_t range[8], nans = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      uint32_t lo = v[0][k], hi = v[0][k], top = v[0][k] & kAbs;
+#pragma unroll
+      for (int j = 1; j < kQTokens; ++j) {
+        lo = pk_min(lo, v[j][k]);
+        hi = pk_max(hi, v[j][k]);
+        top = pk_max_u16(top, v[j][k] & kAbs);
+      }
+      range[2 * k] = __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ kNegHigh;
+      range[2 * k + 1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ kNegHigh;
+      nans |= ((top & 0xffffu) > 0x7c00u ? 1u : 0u) << (2 * k);
+      nans |= (top > 0x7c00ffffu ? 2u : 0u) << (2 * k);
+    }
+    for (int m = 1; m < lanes; m <<= 1) {
+      nans |= __shfl_xor(nans, m * CL);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) range[i] = pk_min(range[i], __shfl_xor(range[i], m * CL));
+    }
+    const int64_t meta = static_cast<int64_t>(bt0 / p.group) * p.C + c0;
+    const bool lead = nv > 0 && bt0 % p.group == 0;
+    each<8>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      const Group g = make_group(range[i], (nans >> i) & 1, p.inv_levels);
+      if (lead) {
+        p.scale[0][meta + i] = half_bits(g.scale);
+        p.zero[0][meta + i] = half_bits(g.zero);
+      }
+      each<kQTokens>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        run[i].template put<j>(
+            kivi_symbol(i & 1 ? high_half(v[j][i >> 1]) : low_half(v[j][i >> 1]), g));
+      });
+    });
+  } else {
+    const int lanes = p.group / 8;  // channel lanes of a group
+    uint32_t range[kQTokens], nans = 0;
+#pragma unroll
+    for (int j = 0; j < kQTokens; ++j) {
+      const uint32_t lo = pk_min(pk_min(v[j][0], v[j][1]), pk_min(v[j][2], v[j][3]));
+      const uint32_t hi = pk_max(pk_max(v[j][0], v[j][1]), pk_max(v[j][2], v[j][3]));
+      const uint32_t top = pk_max_u16(pk_max_u16(v[j][0] & kAbs, v[j][1] & kAbs),
+                                      pk_max_u16(v[j][2] & kAbs, v[j][3] & kAbs));
+      range[j] = pk_min(__builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ kNegHigh,
+                        __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ kNegHigh);
+      nans |= ((top & 0xffffu) > 0x7c00u || top > 0x7c00ffffu ? 1u : 0u) << j;
+    }
+    for (int m = 1; m < lanes; m <<= 1) {
+      nans |= __shfl_xor(nans, m);
+#pragma unroll
+      for (int j = 0; j < kQTokens; ++j) range[j] = pk_min(range[j], __shfl_xor(range[j], m));
+    }
+    const bool lead = chan_ok && c0 % p.group == 0;
+    const int64_t meta = static_cast<int64_t>(bt0) * p.vgroups + c0 / p.group;
+    each<kQTokens>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      const Group g = make_group(range[j], (nans >> j) & 1, p.inv_levels);
+      if (lead && j < nv) {
+        p.scale[1][meta + static_cast<int64_t>(j) * p.vgroups] = half_bits(g.scale);
+        p.zero[1][meta + static_cast<int64_t>(j) * p.vgroups] = half_bits(g.zero);
+      }
+      each<8>([&](auto ic) {
+        constexpr int i = decltype(ic)::value;
+        run[i].template put<j>(
+            kivi_symbol(i & 1 ? high_half(v[j][i >> 1]) : low_half(v[j][i >> 1]), g));
+      });
+    });
   }
   if (nv == 0) return;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int64_t plane = HALF == 0 ? static_cast<int64_t>(d0 + i) * p.H + h : c0 + i;
-    store_run<SB>(p.stream[HALF], plane * p.body + bt0, sym[i], nv);
+    store_run<W, BYTES>(p.stream[HALF], plane * p.body + bt0, run[i], nv);
   }
 }
 
-template <int DT, int SB>
+template <int DT, int W, bool BYTES>
 __global__ __launch_bounds__(kQThreads) void kivi_quantize_kernel(KiviQuantParams p) {
   uint32_t tile = blockIdx.x;
   if (tile < static_cast<uint32_t>(p.tiles[0])) {
-    kivi_quantize_tile<0, DT, SB>(p, tile);
+    kivi_quantize_tile<0, DT, W, BYTES>(p, tile);
     return;
   }
   tile -= p.tiles[0];
   if (tile < static_cast<uint32_t>(p.tiles[1])) {
-    kivi_quantize_tile<1, DT, SB>(p, tile);
+    kivi_quantize_tile<1, DT, W, BYTES>(p, tile);
     return;
   }
   // sink rows of both halves, 8 channels per thread, and the pad bytes
@@ -447,15 +519,17 @@ __global__ __launch_bounds__(kQThreads) void kivi_quantize_kernel(KiviQuantParam
 }
 
 template <int DT>
-int launch_kivi(const KiviQuantParams& p, int sb, hipStream_t stream) {
+int launch_kivi(const KiviQuantParams& p, int sb, bool bytes, hipStream_t stream) {
   const uint32_t sink_tiles = (2 * p.sink * (p.C / 8) + kQThreads - 1) / kQThreads;
   const dim3 grid(p.tiles[0] + p.tiles[1] + (sink_tiles > 0 ? sink_tiles : 1)), block(kQThreads);
-  switch (sb) {
-    case 0: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 0>), grid, block, 0, stream, p); break;
-    case 2: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 2>), grid, block, 0, stream, p); break;
-    case 4: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 4>), grid, block, 0, stream, p); break;
-    default: hipLaunchKernelGGL((kivi_quantize_kernel<DT, 8>), grid, block, 0, stream, p); break;
-  }
+  if (bytes)
+    hipLaunchKernelGGL((kivi_quantize_kernel<DT, 8, true>), grid, block, 0, stream, p);
+  else if (sb == 2)
+    hipLaunchKernelGGL((kivi_quantize_kernel<DT, 2, false>), grid, block, 0, stream, p);
+  else if (sb == 4)
+    hipLaunchKernelGGL((kivi_quantize_kernel<DT, 4, false>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((kivi_quantize_kernel<DT, 8, false>), grid, block, 0, stream, p);
   return check_launch("kivi_quantize_kernel");
 }
 
@@ -589,8 +663,7 @@ int origami_kivi_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t
   p.C = static_cast<int32_t>(C);
   p.group = static_cast<int32_t>(group_size);
   p.vgroups = static_cast<int32_t>(value_groups);
-  p.levels = static_cast<float>((1 << bits) - 1);
-  p.inv_levels = 1.0f / p.levels;
+  p.inv_levels = 1.0f / static_cast<float>((1 << bits) - 1);
   int64_t grid = 0;
   for (int i = 0; i < 2; ++i) {
     p.stream[i] = direct ? payload + offsets[i] : workspace + i * C * body;
@@ -607,14 +680,13 @@ int origami_kivi_quantize(const void* kv, int64_t dtype, int64_t tokens, int64_t
       2 * sink_tokens * (C / 8) > INT32_MAX)
     return fail(ORIGAMI_ERR_UNSUPPORTED, "KIVI layer exceeds the launch grid");
   const hipStream_t stream = reinterpret_cast<hipStream_t>(stream_);
-  const int store = direct ? sb : 0;
   int rc = ORIGAMI_OK;
   if (dtype == ORIGAMI_DTYPE_FLOAT32)
-    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT32>(p, store, stream);
+    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT32>(p, sb, !direct, stream);
   else if (dtype == ORIGAMI_DTYPE_BFLOAT16)
-    rc = launch_kivi<ORIGAMI_DTYPE_BFLOAT16>(p, store, stream);
+    rc = launch_kivi<ORIGAMI_DTYPE_BFLOAT16>(p, sb, !direct, stream);
   else
-    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT16>(p, store, stream);
+    rc = launch_kivi<ORIGAMI_DTYPE_FLOAT16>(p, sb, !direct, stream);
   for (int i = 0; i < 2 && !direct && rc == ORIGAMI_OK; ++i)
     rc = launch_pack_runs(workspace, &runs[i], 1, sb, payload, stream);
   return rc;
