@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -436,6 +437,9 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef unsigned int u32x3a4 __attribute__((ext_vector_type(3), aligned(4)));
 typedef unsigned int u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x4a1 __attribute__((ext_vector_type(4), aligned(1)));
+typedef unsigned int u32x2a1 __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned int u32a1 __attribute__((aligned(1)));
 
 // How the row kernels address a lane's run of 16 packed symbols (2 * b bytes
 // at bit P of the stream).
@@ -463,6 +467,27 @@ enum RowsMode : int {
   kRowsBits = 9,
 };
 
+// Division of n < 2^31 by a divisor the host knows: n / d = (n + mulhi(n, mul)) >> shift
+// (Granlund and Montgomery's multiply by a rounded-up reciprocal).  The kernels divide
+// tile indices and tokens; the compiler's 64-bit divisions were some 1000 of a restore
+// kernel's instructions before its first load, which a launch of a few waves per CU
+// waits for.
+struct FastDiv {
+  uint32_t mul, shift, d;
+};
+
+FastDiv fast_div(int64_t d) {
+  FastDiv f{0, 0, static_cast<uint32_t>(d)};
+  while ((uint64_t(1) << f.shift) < f.d) ++f.shift;
+  f.mul = static_cast<uint32_t>(
+      ((uint64_t(1) << 32) * ((uint64_t(1) << f.shift) - f.d)) / f.d + 1);
+  return f;
+}
+
+__device__ __forceinline__ uint32_t operator/(uint32_t n, const FastDiv& f) {
+  return (__umulhi(n, f.mul) + n) >> f.shift;
+}
+
 struct RowsParams {
   uint8_t* stream;           // 4-byte aligned base of the flat stream
   int64_t stream_bytes;      // bytes addressable from `stream`
@@ -483,16 +508,23 @@ struct RowsParams {
   int64_t half_stride;       // rows per half step
   int32_t H;
   int32_t nq;                // C / 16
-  int32_t waves;             // waves per workgroup (16, 8 or 4)
+  int32_t waves;             // waves per workgroup (16, 8, 4, 2 or 1)
   int32_t wq;                // wave tiles along channels per workgroup (1, 2, 4)
   int32_t ws;                // wave tiles along tokens per workgroup (waves / wq)
   int32_t nqt;               // workgroups along channels
   int32_t nst;               // workgroups along tokens
-  int64_t ntiles;            // workgroup tiles; a workgroup loops over tiles
+  // workgroup tiles; a workgroup loops over tiles.  Below 2^31: a tile is at least
+  // 16 KiB of K/V.
+  int64_t ntiles;
   int32_t partial_last;      // the last token tile is partial: order those tiles last
+  uint32_t nfull;            // tiles before the partial ones (single-request launches)
+  FastDiv by_st;             // token tiles of the full tiles
+  FastDiv by_qt, by_h;       // nqt, H
+  FastDiv by_bs;             // bs; d = 0: 64-bit division (bs or row_tokens above 2^31)
   int64_t token0;            // first destination token of the tiles (a multiple of 16)
   int32_t nt_stores;         // staged pack: whole 16-byte chunks as non-temporal stores
-  int32_t own_lines;         // staged pack: each stream line written by one tile (16 waves)
+  int32_t own_lines;         // staged pack: each stream line written by one tile
+  int32_t xcd_run;           // 8-bit pack in place: consecutive tiles per XCD (xcd_run_order)
 };
 
 // Per-request fields of a batched restore (one layer of several requests
@@ -509,6 +541,7 @@ struct RowsRequest {
   int64_t ptile0;  // first partial-token-tile workgroup tile of the request
   int32_t nst;
   int32_t partial;  // 1: the last token tile is partial
+  FastDiv by_st;    // its full token tiles
   int32_t nt;       // aligned16 batches: 1 = non-temporal loads (runs on 128-byte lines)
 };
 
@@ -607,9 +640,48 @@ __device__ __forceinline__ void load_run_dwords(const uint8_t* src, uint32_t* w)
   }
 }
 
+// A lane's 16 plane descriptors: staged in LDS, or (CLOSED) the closed form where the
+// plan has one, which needs neither LDS nor its barriers.  Short launches take it: its
+// chain to the first load is shorter.  Launches of whole-tile and split workgroups keep
+// the descriptors in LDS, whose barriers keep a workgroup's waves together (without
+// them the 32768-token restore ran 54.7 us against 53.0).
+template <bool CLOSED>
+struct LanePlanes {
+  const int64_t* desc;  // CLOSED: null where plane k is at first + k * step
+  int64_t first, step;
+  __device__ __forceinline__ bool closed() const { return CLOSED && !desc; }
+  __device__ __forceinline__ int64_t get(int k) const {
+    return closed() ? first + k * step : desc[k];
+  }
+};
+
+// The NW dwords from byte `byte0` of the stream.  A run whose dwords pass the end takes
+// them one by one, the stream's last dword for those past it: bits past the stream
+// belong to no symbol that is kept.  Its loads go out with the others; loading such a run
+// again, guarded dword by dword, after the others had returned made the one wave that
+// holds the stream's end a serial chain.
+template <int NW>
+__device__ __forceinline__ void load_run(const RowsParams& p, int64_t byte0, uint32_t* w) {
+  if (byte0 + 4 * NW <= p.stream_bytes) {
+    if constexpr (NW == 5) {
+      load_run_dwords<4>(p.stream + byte0, w);
+      load_run_dwords<1>(p.stream + byte0 + 16, w + 4);
+    } else {
+      load_run_dwords<NW>(p.stream + byte0, w);
+    }
+  } else {
+    const int64_t last = (p.stream_bytes - 1) & ~int64_t(3);
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const int64_t at = byte0 + 4 * i;
+      w[i] = *reinterpret_cast<const uint32_t*>(p.stream + (at < last ? at : last));
+    }
+  }
+}
+
 // The window and shift modes of load_planes16 (below).
-template <int BITS, int MODE, bool SERIAL>
-__device__ __forceinline__ void load_runs16(const RowsParams& p, const int64_t* desc,
+template <int BITS, int MODE, bool SERIAL, bool CLOSED>
+__device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlanes<CLOSED>& planes,
                                             int64_t sym0, bool any, uint32_t (&v)[16][4]) {
   static_assert(MODE == kRowsWindow || MODE == kRowsShift, "restore addressing mode");
   constexpr int NU = (16 * BITS + 31) / 32;  // = ceil(b / 2): dwords of a run
@@ -618,129 +690,159 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const int64_t* 
   // kRowsShift: the run starts at any bit, so the NU + 1 dwords from the one
   // holding its first bit hold it.
   constexpr int NW = MODE == kRowsShift ? NU + 1 : NU;
+  auto first_byte = [](int64_t P) {
+    return MODE == kRowsShift ? (P >> 5) * 4 : (P >> 3) & ~int64_t(3);
+  };
+  auto funnel = [](int64_t P) {
+    return MODE == kRowsShift ? static_cast<uint32_t>(P & 31)
+           : (BITS % 2 == 1 && ((P >> 3) & 2)) ? 16u
+                                               : 0u;
+  };
+  auto expand = [&](const uint32_t* w, uint32_t sh, uint32_t (&out)[4]) {
+    uint32_t u[NU > 4 ? NU : 4];
+#pragma unroll
+    for (int i = 0; i < NU; ++i)
+      u[i] = __builtin_amdgcn_alignbit(i + 1 < NW ? w[i + 1] : 0u, w[i], sh);
+    expand16<BITS>(u, out);
+  };
   if constexpr (SERIAL) {
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-      const int64_t d = desc[k];
+      const int64_t d = planes.get(k);
       v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0;
       if (d < 0 || !any) continue;
       const int64_t P = d + p.bit_bias + sym0 * BITS;
-      const int64_t byte0 = MODE == kRowsShift ? (P >> 5) * 4 : (P >> 3) & ~int64_t(3);
-      uint32_t w[NU + 1], u[NU > 4 ? NU : 4];
-      uint32_t sh;
-      if (byte0 + 4 * NW <= p.stream_bytes) {
-        if constexpr (NW == 5) {
-          load_run_dwords<4>(p.stream + byte0, w);
-          load_run_dwords<1>(p.stream + byte0 + 16, w + 4);
-        } else {
-          load_run_dwords<NW>(p.stream + byte0, w);
-        }
-        if constexpr (NW == NU) w[NU] = 0;
-        sh = MODE == kRowsShift ? static_cast<uint32_t>(P & 31)
-             : (BITS % 2 == 1 && ((P >> 3) & 2)) ? 16u
-                                                 : 0u;
-      } else {  // as below: the NU + 1 dwords from the one holding bit P
-        const int64_t d0 = P >> 5;
-        sh = static_cast<uint32_t>(P & 31);
-#pragma unroll
-        for (int i = 0; i <= NU; ++i)
-          w[i] = load_dword_guarded(p.stream, (d0 + i) * 4, p.stream_bytes);
-      }
-#pragma unroll
-      for (int i = 0; i < NU; ++i) u[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], sh);
-      expand16<BITS>(u, v[k]);
+      uint32_t w[NW];
+      load_run<NW>(p, first_byte(P), w);
+      expand(w, funnel(P), v[k]);
     }
   } else {
     uint32_t w[16][NW];
-    uint32_t tail = 0;    // bit k: plane k's dwords pass the end of the stream
     uint32_t shp[4] = {};  // byte k & 3 of shp[k >> 2]: plane k's funnel shift
+    // Planes in order, each of at least 32 bytes (a run and its dwords): only the dwords
+    // of the last plane's run can pass the end of the stream.  Its lanes take the
+    // stream's last NW dwords and move them down to their own afterwards, so that no
+    // lane's loads wait for another's (in a branch of their own they did).  A lane past
+    // the tokens, whose symbols the shift mode clears, loads its planes' first runs.
+    const int64_t P0 = planes.first + p.bit_bias + (any ? sym0 * BITS : 0);
+    const int64_t last = ((p.stream_bytes + 3) & ~int64_t(3)) - 4 * NW;
+    if (planes.closed() && planes.step >= 256 && (any || MODE == kRowsShift) && last >= 0) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int64_t d = desc[k];
-#pragma unroll
-      for (int i = 0; i < NW; ++i) w[k][i] = 0;
-      if (d >= 0 && any) {
-        const int64_t P = d + p.bit_bias + sym0 * BITS;
-        const int64_t byte0 = MODE == kRowsShift ? (P >> 5) * 4 : (P >> 3) & ~int64_t(3);
-        const uint32_t sh = MODE == kRowsShift ? static_cast<uint32_t>(P & 31)
-                            : (BITS % 2 == 1 && ((P >> 3) & 2)) ? 16u
-                                                                : 0u;
-        shp[k >> 2] |= sh << (8 * (k & 3));
-        if (byte0 + 4 * NW <= p.stream_bytes) {
-          if constexpr (NW == 5) {
-            load_run_dwords<4>(p.stream + byte0, w[k]);
-            load_run_dwords<1>(p.stream + byte0 + 16, w[k] + 4);
-          } else {
-            load_run_dwords<NW>(p.stream + byte0, w[k]);
-          }
+      for (int k = 0; k < 16; ++k) {
+        const int64_t P = P0 + k * planes.step;
+        int64_t byte0 = first_byte(P);
+        if (k == 15) byte0 = byte0 < last ? byte0 : last;
+        const uint8_t* src = p.stream + byte0;
+        shp[k >> 2] |= funnel(P) << (8 * (k & 3));
+        if constexpr (NW == 5) {
+          load_run_dwords<4>(src, w[k]);
+          load_run_dwords<1>(src + 16, w[k] + 4);
         } else {
-          tail |= 1u << k;
+          load_run_dwords<NW>(src, w[k]);
+        }
+      }
+      const int64_t past = (first_byte(P0 + 15 * planes.step) - last) >> 2;
+      if (past > 0) {
+#pragma unroll
+        for (int m = 1; m < NW; ++m)
+          if (past >= m) {
+#pragma unroll
+            for (int i = 0; i + 1 < NW; ++i) w[15][i] = w[15][i + 1];
+          }
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int64_t d = planes.get(k);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w[k][i] = 0;
+        if (d >= 0 && any) {
+          const int64_t P = d + p.bit_bias + sym0 * BITS;
+          shp[k >> 2] |= funnel(P) << (8 * (k & 3));
+          load_run<NW>(p, first_byte(P), w[k]);
         }
       }
     }
-    // keeps the descriptors from staying live in registers until the tail
-    // reloads below (they are read from LDS again there)
+    // every plane's dwords are requested before any is used
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      uint32_t u[NU > 4 ? NU : 4];
-      if (tail & (1u << k)) {
-        // the NU + 1 dwords from the one holding bit P, those past the end of
-        // the stream read as zeros
-        const int64_t P = desc[k] + p.bit_bias + sym0 * BITS;
-        const int64_t d0 = P >> 5;
-        const uint32_t sh = static_cast<uint32_t>(P & 31);
-        uint32_t t[NU + 1];
-#pragma unroll
-        for (int i = 0; i <= NU; ++i)
-          t[i] = load_dword_guarded(p.stream, (d0 + i) * 4, p.stream_bytes);
-#pragma unroll
-        for (int i = 0; i < NU; ++i) u[i] = __builtin_amdgcn_alignbit(t[i + 1], t[i], sh);
-      } else {
-        const uint32_t sh = (shp[k >> 2] >> (8 * (k & 3))) & 31u;
-#pragma unroll
-        for (int i = 0; i < NU; ++i)
-          u[i] = __builtin_amdgcn_alignbit(i + 1 < NW ? w[k][i + 1] : 0u, w[k][i], sh);
-      }
-      expand16<BITS>(u, v[k]);
-    }
+    for (int k = 0; k < 16; ++k) expand(w[k], (shp[k >> 2] >> (8 * (k & 3))) & 31u, v[k]);
   }
 }
 
 // Loads a lane's 16 symbols of each of its 16 planes (plane k at stream bit
-// P_k = desc[k] + bit_bias + sym0 * b; a plane with desc[k] < 0, or every
+// P_k = planes.get(k) + bit_bias + sym0 * b; a plane whose descriptor is < 0, or every
 // plane when `any` is false, reads as zeros) into v[k], one byte per symbol.
 // Every plane's dwords are requested before any of them is used, so a lane
 // has all 16 loads in flight at once: with the funnel shift of each plane
 // next to its loads, the compiler waited for every plane's data before
 // requesting the next plane's (16 round trips per lane, 2053 tokens restored
-// in 15.9 us against 8.5 for 2048).  A run whose dwords would pass the end
-// of the stream is read again dword by dword afterwards.  SERIAL keeps the
+// in 15.9 us against 8.5 for 2048).  SERIAL keeps the
 // funnel shift next to each plane's loads (window and shift modes): with two
 // loads per plane (b = 7, 8 in shift mode) and more than 12 waves per CU that
 // order restored faster (15000 tokens 28.2 us, against 30.5 with every load
 // in flight).
-template <int BITS, int MODE, bool SERIAL = false>
-__device__ __forceinline__ void load_planes16(const RowsParams& p, const int64_t* desc,
-                                              int64_t sym0, bool any, uint32_t (&v)[16][4]) {
+template <int BITS, int MODE, bool SERIAL = false, bool CLOSED = false>
+__device__ __forceinline__ void load_planes16(const RowsParams& p,
+                                              const LanePlanes<CLOSED>& planes, int64_t sym0,
+                                              bool any, uint32_t (&v)[16][4]) {
   if constexpr (MODE == kRowsAligned16 || MODE == kRowsAligned16Cached) {
     static_assert(BITS == 8, "aligned loads are for 8-bit symbols");
+    auto load = [&](int k, const uint8_t* at) {
+      // the stream is read once: non-temporal when each 8-lane run is one line
+      const u32x4* src = reinterpret_cast<const u32x4*>(at);
+      const u32x4 x = MODE == kRowsAligned16 ? __builtin_nontemporal_load(src) : *src;
+      v[k][0] = x.x;
+      v[k][1] = x.y;
+      v[k][2] = x.z;
+      v[k][3] = x.w;
+    };
+    if (planes.closed() && any) {
+      const uint8_t* at = p.stream + ((planes.first + p.bit_bias + sym0 * 8) >> 3);
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int64_t d = desc[k];
-      v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0;
-      if (d >= 0 && any) {
-        // the stream is read once: non-temporal when each 8-lane run is one line
-        const u32x4* src = reinterpret_cast<const u32x4*>(p.stream + ((d + p.bit_bias + sym0 * 8) >> 3));
-        const u32x4 x = MODE == kRowsAligned16 ? __builtin_nontemporal_load(src) : *src;
-        v[k][0] = x.x;
-        v[k][1] = x.y;
-        v[k][2] = x.z;
-        v[k][3] = x.w;
+      for (int k = 0; k < 16; ++k) load(k, at + k * (planes.step >> 3));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int64_t d = planes.get(k);
+        v[k][0] = v[k][1] = v[k][2] = v[k][3] = 0;
+        if (d >= 0 && any) load(k, p.stream + ((d + p.bit_bias + sym0 * 8) >> 3));
       }
     }
   } else {
-    load_runs16<BITS, MODE, SERIAL>(p, desc, sym0, any, v);
+    load_runs16<BITS, MODE, SERIAL, CLOSED>(p, planes, sym0, any, v);
+  }
+}
+
+// The dword of c holding byte j (0 <= j < 16), by selects on scalars (an
+// indexed read of c would put it in scratch memory).
+__device__ __forceinline__ uint32_t chunk_word(uint32_t c0, uint32_t c1, uint32_t c2,
+                                               uint32_t c3, int j) {
+  const uint32_t lo = (j & 4) ? c1 : c0, hi = (j & 4) ? c3 : c2;
+  return (j & 8) ? hi : lo;
+}
+
+// Writes the first n (1..16) bytes of u[0..3] to dst, at any byte address, in one store
+// or two that overlap.
+__device__ __forceinline__ void store_bytes16(uint8_t* dst, const uint32_t* u, int n) {
+  // the dword at byte m (0 <= m <= 12) of u
+  auto at = [&](int m) {
+    const uint32_t lo = chunk_word(u[0], u[1], u[2], u[3], m);
+    const uint32_t hi = chunk_word(u[1], u[2], u[3], u[3], m);
+    return __builtin_amdgcn_alignbyte(hi, lo, m & 3);
+  };
+  if (n == 16) {
+    *reinterpret_cast<u32x4a1*>(dst) = u32x4a1{u[0], u[1], u[2], u[3]};
+  } else if (n >= 8) {
+    *reinterpret_cast<u32x2a1*>(dst) = u32x2a1{u[0], u[1]};
+    *reinterpret_cast<u32x2a1*>(dst + n - 8) = u32x2a1{at(n - 8), at(n - 4)};
+  } else if (n >= 4) {
+    *reinterpret_cast<u32a1*>(dst) = u[0];
+    *reinterpret_cast<u32a1*>(dst + n - 4) = at(n - 4);
+  } else {
+    dst[0] = static_cast<uint8_t>(u[0]);
+    if (n > 1) dst[1] = static_cast<uint8_t>(u[0] >> 8);
+    if (n > 2) dst[2] = static_cast<uint8_t>(u[0] >> 16);
   }
 }
 
@@ -790,6 +892,10 @@ __device__ __forceinline__ void store_stream(uint8_t* dst, const uint32_t* u, in
     ORIGAMI_RUN_STORE(uint16_t, d[NU - 1], half);
   } else {
     static_assert(MODE == kRowsBytes, "pack modes: aligned16, window, bytes");
+    if constexpr (BITS == 8) {
+      store_bytes16(dst, u, nbytes);
+      return;
+    }
     // nbytes <= 2b bytes at any byte address: up to 3 head bytes to the next
     // dword, whole dwords, then up to 3 tail bytes.  Byte j of the run is
     // byte j & 3 of u[j >> 2].
@@ -837,22 +943,24 @@ struct TileCoord {
 // last token tile is partial, the full token tiles of every (channel tile,
 // head, half) come first and the partial ones after them, so that the small
 // tiles finish the launch instead of unbalancing its full rounds.
-// A tile is its token tile `st` and the rest (channel tile fastest, then
-// head, then half).
+// A tile is its token tile `st`, channel tile `qt` (the fastest of the rest), head and
+// half.
 struct TileIndex {
-  int st;
-  int64_t rest;
+  int st, qt, h, half;
 };
 
+__device__ __forceinline__ TileIndex tile_index(const RowsParams& p, int st, uint32_t rest) {
+  const uint32_t hq = rest / p.by_qt, half = hq / p.by_h;
+  return {st, static_cast<int>(rest - hq * p.by_qt.d), static_cast<int>(hq - half * p.by_h.d),
+          static_cast<int>(half)};
+}
+
 // Splits a tile index of a single-request launch.
-__device__ __forceinline__ TileIndex split_tile(const RowsParams& p, int64_t tile) {
-  if (p.partial_last) {
-    const int full = p.nst - 1;
-    const int64_t nfull = p.ntiles / p.nst * full;
-    if (tile >= nfull) return {full, tile - nfull};
-    return {static_cast<int>(tile % full), tile / full};
-  }
-  return {static_cast<int>(tile % p.nst), tile / p.nst};
+__device__ __forceinline__ TileIndex split_tile(const RowsParams& p, int64_t index) {
+  const uint32_t tile = static_cast<uint32_t>(index);
+  if (p.partial_last && tile >= p.nfull) return tile_index(p, p.nst - 1, tile - p.nfull);
+  const uint32_t rest = tile / p.by_st;
+  return tile_index(p, static_cast<int>(tile - rest * p.by_st.d), rest);
 }
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup b runs on XCD
@@ -875,27 +983,23 @@ __device__ __forceinline__ int64_t xcd_run_order(int64_t i, int64_t n, int run) 
 template <bool SPLIT = false, int SEG = kSegTokens>
 __device__ __forceinline__ TileCoord tile_coord(const RowsParams& p, TileIndex ti,
                                                 int slice = 0) {
-  const int st = ti.st;
-  int64_t tile = ti.rest;
-  const int qt = static_cast<int>(tile % p.nqt);
-  tile /= p.nqt;
   TileCoord tc;
-  tc.h = static_cast<int>(tile % p.H);
-  tc.half = static_cast<int>(tile / p.H);
+  tc.h = ti.h;
+  tc.half = ti.half;
   const int lane = threadIdx.x & 63;
   int wqi, wsi;
   if constexpr (SPLIT) {
     const int wave = slice * kRowsSplitWaves + (threadIdx.x >> 6);
-    wqi = wave / p.ws;
-    wsi = wave % p.ws;
+    wqi = wave >= p.ws ? 1 : 0;  // wq <= kRowsWq = 2
+    wsi = wave - (wqi ? p.ws : 0);
   } else {
     const int wave = threadIdx.x >> 6;
-    wqi = wave % p.wq;
-    wsi = wave / p.wq;
+    wsi = p.wq == 2 ? wave >> 1 : wave;
+    wqi = p.wq == 2 ? wave & 1 : 0;
   }
   tc.slot = wqi * kLaneGroups + (lane >> 3);
-  tc.q = qt * p.wq * kLaneGroups + tc.slot;
-  tc.t0 = p.token0 + (static_cast<int64_t>(st * p.ws + wsi) * kLaneSegs + (lane & 7)) * SEG;
+  tc.q = ti.qt * p.wq * kLaneGroups + tc.slot;
+  tc.t0 = p.token0 + (static_cast<int64_t>(ti.st * p.ws + wsi) * kLaneSegs + (lane & 7)) * SEG;
   return tc;
 }
 
@@ -904,16 +1008,22 @@ __device__ __forceinline__ TileCoord tile_coord(const RowsParams& p, TileIndex t
 // is still reading.
 __device__ __forceinline__ void load_descriptors(const RowsParams& p, TileIndex ti,
                                                  int64_t* desc) {
-  const int qt = static_cast<int>(ti.rest % p.nqt);
-  const int h = static_cast<int>((ti.rest / p.nqt) % p.H);
   const int n = p.wq * kWavePlanes;
   __syncthreads();
   for (int i = static_cast<int>(threadIdx.x); i < n; i += static_cast<int>(blockDim.x)) {
-    const int64_t c = static_cast<int64_t>(qt) * n + i;
-    const int64_t plane = static_cast<int64_t>(h) * p.C + c;
+    const int64_t c = static_cast<int64_t>(ti.qt) * n + i;
+    const int64_t plane = static_cast<int64_t>(ti.h) * p.C + c;
     desc[i] = c >= p.C ? -1 : p.planes ? p.planes[plane] : p.plane_base + plane * p.plane_bits;
   }
   __syncthreads();
+}
+
+template <bool CLOSED>
+__device__ __forceinline__ LanePlanes<CLOSED> lane_planes(const RowsParams& p, const TileCoord& tc,
+                                                  const int64_t* desc) {
+  if (!CLOSED || p.planes) return {desc + tc.slot * 16, 0, 0};
+  const int64_t plane = static_cast<int64_t>(tc.h) * p.C + static_cast<int64_t>(tc.q) * 16;
+  return {nullptr, p.plane_base + plane * p.plane_bits, p.plane_bits};
 }
 
 // Row cursor over the 16 tokens of a lane: follows the block table.
@@ -923,7 +1033,7 @@ struct RowCursor {
 
 __device__ __forceinline__ void cursor_init(const RowsParams& p, int64_t t0, RowCursor& rc) {
   if (p.block_ids) {
-    rc.blk = t0 / p.bs;
+    rc.blk = p.by_bs.d ? static_cast<uint32_t>(t0) / p.by_bs : t0 / p.bs;
     rc.off = t0 - rc.blk * p.bs;
     rc.pid = p.block_ids[rc.blk];
   } else {
@@ -950,7 +1060,9 @@ __device__ __forceinline__ int64_t cursor_row(const RowsParams& p, int half, con
   return rc.pid * p.blk_stride + half * p.half_stride + rc.off;
 }
 
-// Calls f(j, row) for each token t0 + j (t0 % 16 == 0, j < 16 and j < nrows)
+// Calls f(j, row) for each token t0 + j (t0 % 16 == 0, j < 16 and j < nrows), `rc` the
+// cursor of token t0 (its table entry is requested when the cursor is made, so a caller
+// that makes it before its stream loads waits once for both)
 // whose block is in the cache, with its row index.  ONEBLK: every block holds
 // a multiple of 16 rows, or there is no block table, so the 16 tokens are
 // consecutive rows of one block: one table load, then fixed strides.
@@ -962,17 +1074,22 @@ __device__ __forceinline__ int64_t cursor_row(const RowsParams& p, int half, con
 // HBM peak) and launches of few waves per CU up to half their time, while
 // whole-tile launches of 8 or more waves per CU run 1-4% faster with it: the
 // host picks by launch size (waves_per_cu).
-template <bool ONEBLK, class F>
-__device__ __forceinline__ void for_rows16(const RowsParams& p, int half, int64_t t0,
+// SHORT: all 16 rows without a check each where the lane has them (launches of few waves
+// per CU; the split restores are 0.5% faster with the checks between their stores).
+template <bool ONEBLK, bool SHORT, class F>
+__device__ __forceinline__ void for_rows16(const RowsParams& p, int half, RowCursor rc,
                                            int64_t nrows, F&& f) {
-  RowCursor rc;
-  cursor_init(p, t0, rc);
   if constexpr (ONEBLK) {
     const int64_t row0 = cursor_row(p, half, rc);
     if (row0 < 0) return;
+    if (SHORT && nrows >= 16) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-      if (j < nrows) f(j, row0 + j);
+      for (int j = 0; j < 16; ++j) f(j, row0 + j);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (j < nrows) f(j, row0 + j);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
@@ -997,8 +1114,12 @@ __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
   const int64_t nv = p.T - tc.t0;  // tokens of this segment that hold symbols
   const int64_t sym0 = static_cast<int64_t>(tc.half) * p.T + tc.t0;
 
+  constexpr bool kShort = ONEBLK && !SPLIT;
+  RowCursor rc;
+  if constexpr (kShort) cursor_init(p, tc.t0, rc);
   uint32_t v[16][4];
-  load_planes16<BITS, MODE, SERIAL>(p, desc + tc.slot * 16, sym0, nv > 0, v);
+  load_planes16<BITS, MODE, SERIAL>(p, lane_planes<kShort>(p, tc, desc), sym0, nv > 0, v);
+  if constexpr (!kShort) cursor_init(p, tc.t0, rc);
   if (MODE == kRowsShift && nv < 16) {  // other modes: T % 16 == 0
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -1015,7 +1136,7 @@ __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
 
   uint8_t* col = p.rows + static_cast<int64_t>(tc.h) * p.head_pitch + tc.q * 16;
   // each row is written once: non-temporal
-  for_rows16<ONEBLK>(p, tc.half, tc.t0, p.row_tokens - tc.t0, [&](int j, int64_t row) {
+  for_rows16<ONEBLK, kShort>(p, tc.half, rc, p.row_tokens - tc.t0, [&](int j, int64_t row) {
     const u32x4 x = {o[j][0], o[j][1], o[j][2], o[j][3]};
     __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(col + row * p.row_pitch));
   });
@@ -1028,7 +1149,7 @@ __global__ __launch_bounds__(kRowsThreads) void rows_unpack_kernel(RowsParams p)
   __shared__ int64_t desc[kTilePlanes];
   for (int64_t tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
     const TileIndex ti = split_tile(p, tile);
-    load_descriptors(p, ti, desc);
+    if (!ONEBLK || p.planes) load_descriptors(p, ti, desc);
     unpack_tile<BITS, MODE, false, ONEBLK, SERIAL>(p, ti, desc);
   }
 }
@@ -1066,10 +1187,11 @@ __device__ __forceinline__ void unpack_tile_wide(const RowsParams& p, TileIndex 
   const bool has_symbols = tc.t0 < p.T;
   const int64_t sym0 = static_cast<int64_t>(tc.half) * p.T + tc.t0;
 
+  const LanePlanes<ONEBLK> planes = lane_planes<ONEBLK>(p, tc, desc);
   uint32_t w[16][4];
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    const int64_t d = desc[tc.slot * 16 + k];
+    const int64_t d = planes.get(k);
     w[k][0] = w[k][1] = w[k][2] = w[k][3] = 0;
     if (d >= 0 && has_symbols) {
       const u32x4* src = reinterpret_cast<const u32x4*>(p.stream + ((d + p.bit_bias + sym0 * BITS) >> 3));
@@ -1102,7 +1224,9 @@ __device__ __forceinline__ void unpack_tile_wide(const RowsParams& p, TileIndex 
     }
     uint32_t o[16][4];
     transpose16(v, o);
-    for_rows16<ONEBLK>(p, tc.half, t0, p.row_tokens - t0, [&](int j, int64_t row) {
+    RowCursor rc;
+    cursor_init(p, t0, rc);
+    for_rows16<ONEBLK, ONEBLK>(p, tc.half, rc, p.row_tokens - t0, [&](int j, int64_t row) {
       const u32x4 x = {o[j][0], o[j][1], o[j][2], o[j][3]};
       __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(col + row * p.row_pitch));
     });
@@ -1118,7 +1242,7 @@ __global__ __launch_bounds__(kWideMaxWaves * 64) void rows_unpack_wide_kernel(Ro
   __shared__ int64_t desc[kTilePlanes];
   for (int64_t tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
     const TileIndex ti = split_tile(p, tile);
-    load_descriptors(p, ti, desc);
+    if (!ONEBLK || p.planes) load_descriptors(p, ti, desc);
     unpack_tile_wide<BITS, NT, ONEBLK>(p, ti, desc);
   }
 }
@@ -1136,12 +1260,13 @@ __device__ __forceinline__ void batch_tile(const RowsBatch& b, int64_t tile, int
   TileIndex ti;
   if (tile < b.nfull) {
     while (r + 1 < b.nreq && tile >= b.req[r + 1].tile0) ++r;
-    const int full = b.req[r].nst - b.req[r].partial;
-    const int64_t local = tile - b.req[r].tile0;
-    ti = {static_cast<int>(local % full), local / full};
+    const uint32_t local = static_cast<uint32_t>(tile - b.req[r].tile0);
+    const uint32_t rest = local / b.req[r].by_st;
+    ti = tile_index(b.common, static_cast<int>(local - rest * b.req[r].by_st.d), rest);
   } else {
     while (r + 1 < b.nreq && tile >= b.req[r + 1].ptile0) ++r;
-    ti = {b.req[r].nst - 1, tile - b.req[r].ptile0};
+    ti = tile_index(b.common, b.req[r].nst - 1,
+                    static_cast<uint32_t>(tile - b.req[r].ptile0));
   }
   const RowsRequest& q = b.req[r];
   RowsParams p = b.common;
@@ -1156,7 +1281,7 @@ __device__ __forceinline__ void batch_tile(const RowsBatch& b, int64_t tile, int
   p.row_tokens = q.row_tokens;
   p.nst = q.nst;
   p.token0 = q.token0;
-  load_descriptors(p, ti, desc);
+  if (SPLIT || !ONEBLK || p.planes) load_descriptors(p, ti, desc);
   if constexpr (MODE == kRowsAligned16) {
     // one launch for the batch, the load policy per request
     if (q.nt)
@@ -1182,9 +1307,14 @@ __global__ __launch_bounds__(kRowsSplitWaves * 64) void rows_unpack_batch_split_
     RowsBatch b, int sh) {
   __shared__ int64_t desc[kTilePlanes];
   const int64_t slots = b.common.ntiles << sh;
-  for (int64_t s = blockIdx.x; s < slots; s += gridDim.x)
+  for (int64_t i = blockIdx.x; i < slots; i += gridDim.x) {
+    // pairs of slices, which share stream lines off 128-byte lines, on one XCD: the
+    // 8-request Qwen2.5-7B batch 135.2 us with runs of 1, 134.0 of 2, 134.5 of 4, 135.0
+    // of 16
+    const int64_t s = xcd_run_order(i, slots, 2);
     batch_tile<BITS, MODE, true, ONEBLK, false>(b, s >> sh, desc,
                                                static_cast<int>(s & ((1 << sh) - 1)));
+  }
 }
 
 // Calls f(std::integral_constant<int, i>) for i = 0 .. N - 1, in order.
@@ -1194,14 +1324,6 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for<N - 1>(f);
     f(std::integral_constant<int, N - 1>{});
   }
-}
-
-// The dword of c holding byte j (0 <= j < 16), by selects on scalars (an
-// indexed read of c would put it in scratch memory).
-__device__ __forceinline__ uint32_t chunk_word(uint32_t c0, uint32_t c1, uint32_t c2,
-                                               uint32_t c3, int j) {
-  const uint32_t lo = (j & 4) ? c1 : c0, hi = (j & 4) ? c3 : c2;
-  return (j & 8) ? hi : lo;
 }
 
 // Writes bytes [lo, hi) of the 16-byte aligned chunk at dst (0 <= lo < hi
@@ -1238,7 +1360,7 @@ __device__ __forceinline__ void store_chunk_part(uint8_t* dst, uint32_t c0, uint
 // 16-byte channel column) through the block table; missing rows read as 0.
 // ONEBLK as for for_rows16: without it the row loads are requested one after
 // another, which is faster only in launches of more than 12 waves per CU
-// (6 for the staged pack).
+// (in the staged pack always, which runs at 8 or more).
 template <bool ONEBLK>
 __device__ __forceinline__ void load_tile_rows(const RowsParams& p, const TileCoord& tc, int nv,
                                                uint32_t (&r)[16][4]) {
@@ -1246,7 +1368,9 @@ __device__ __forceinline__ void load_tile_rows(const RowsParams& p, const TileCo
 #pragma unroll
   for (int j = 0; j < 16; ++j) r[j][0] = r[j][1] = r[j][2] = r[j][3] = 0;
   if (nv <= 0) return;
-  for_rows16<ONEBLK>(p, tc.half, tc.t0, nv, [&](int j, int64_t row) {
+  RowCursor rc;
+  cursor_init(p, tc.t0, rc);
+  for_rows16<ONEBLK, ONEBLK>(p, tc.half, rc, nv, [&](int j, int64_t row) {
     const u32x4 x =
         __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(col + row * p.row_pitch));
     r[j][0] = x.x;
@@ -1269,12 +1393,11 @@ __device__ __forceinline__ void load_tile_rows(const RowsParams& p, const TileCo
 // buffers, so one barrier per round separates writers and readers.
 constexpr int kStagePlanes = 4;
 constexpr int kStageFront = 16, kStageBack = 32;  // pad bytes around a region
-// A round: kStagePlanes x (wq * 8 slots) regions of ws * 128 + pad bytes, for
-// a workgroup of `waves` waves.
-constexpr int stage_round_bytes(int waves) {
-  return kStagePlanes * (waves * 1024 + kRowsWq * kLaneGroups * (kStageFront + kStageBack));
-}
-static_assert(2 * stage_round_bytes(kRowsMaxWaves) + kRowsWq * kWavePlanes * 8 <= 160 * 1024,
+// A round: kStagePlanes x 8 slots (one wave tile along channels) regions of 16 * 128 +
+// pad bytes.
+constexpr int kStageRoundBytes =
+    kStagePlanes * kLaneGroups * (kRowsMaxWaves * 128 + kStageFront + kStageBack);
+static_assert(2 * kStageRoundBytes + kRowsWq * kWavePlanes * 8 <= 160 * 1024,
               "LDS of the staged pack");
 
 // Writes this lane's 16-byte chunk of region line j: stream bytes
@@ -1309,7 +1432,6 @@ __device__ __forceinline__ void store_region_chunk(uint8_t* line0, const uint8_t
 // Every wave of the workgroup runs this for every tile (no early exit: the
 // rounds hold barriers); lanes outside the tile's channels or tokens only
 // take part in the barriers.
-template <int WAVES, bool ONEBLK>
 __device__ __forceinline__ void pack_tile_staged8(const RowsParams& p, TileIndex ti,
                                                   const int64_t* desc, uint8_t* stage) {
   const TileCoord tc = tile_coord(p, ti);
@@ -1321,7 +1443,7 @@ __device__ __forceinline__ void pack_tile_staged8(const RowsParams& p, TileIndex
   const int nv = run_ok ? static_cast<int>(p.T - tc.t0 < 16 ? p.T - tc.t0 : 16) : 0;
 
   uint32_t r[16][4];
-  load_tile_rows<ONEBLK>(p, tc, nv, r);
+  load_tile_rows<false>(p, tc, nv, r);
   uint32_t v[16][4];
   transpose16(r, v);
 
@@ -1332,7 +1454,7 @@ __device__ __forceinline__ void pack_tile_staged8(const RowsParams& p, TileIndex
   const int run_off = kStageFront + (wsi * kLaneSegs + s) * kSegTokens;
   static_for<16 / kStagePlanes>([&](auto rc) {
     constexpr int round = decltype(rc)::value;
-    uint8_t* const buf = stage + (round & 1) * stage_round_bytes(WAVES);
+    uint8_t* const buf = stage + (round & 1) * kStageRoundBytes;
     static_for<kStagePlanes>([&](auto kc) {
       constexpr int kk = decltype(kc)::value, k = round * kStagePlanes + kk;
       if (run_ok && desc[tc.slot * 16 + k] >= 0)
@@ -1407,7 +1529,6 @@ __device__ __forceinline__ void store_owned_chunk(uint8_t* line0, const uint8_t*
 // 8 or more waves per CU, where the walk is the faster order anyway).
 __device__ __forceinline__ void pack_tile_owned(const RowsParams& p, TileIndex ti,
                                                 const int64_t* desc, uint8_t* stage) {
-  constexpr int WAVES = 16;
   TileCoord tc = tile_coord(p, ti);
   const int s = static_cast<int>(threadIdx.x & 7);
   const int wsi = static_cast<int>(threadIdx.x >> 6);  // wq == 1: the wave's token row
@@ -1435,14 +1556,14 @@ __device__ __forceinline__ void pack_tile_owned(const RowsParams& p, TileIndex t
   const int n = static_cast<int>(p.T - T0 < kOwnTokens ? p.T - T0 : kOwnTokens);
   const bool first_part = half == 0 && T0 == 0;         // the plane's first line
   const bool last_part = half == 1 && T0 + n == p.T;    // the plane's last line
-  const int RS = WAVES * 128 + kStageFront + kStageBack;
+  const int RS = kRowsMaxWaves * 128 + kStageFront + kStageBack;
   const int slots = p.wq * kLaneGroups;
   const int64_t sym0 = half * p.T + T0;
   const int run_off = kStageFront + (wsi * kLaneSegs + s) * kSegTokens;
   const bool nt = p.nt_stores != 0;
   static_for<16 / kStagePlanes>([&](auto rc) {
     constexpr int round = decltype(rc)::value;
-    uint8_t* const buf = stage + (round & 1) * stage_round_bytes(WAVES);
+    uint8_t* const buf = stage + (round & 1) * kStageRoundBytes;
     static_for<kStagePlanes>([&](auto kc) {
       constexpr int kk = decltype(kc)::value, k = round * kStagePlanes + kk;
       if (nv > 0 && desc[tc.slot * 16 + k] >= 0)
@@ -1524,9 +1645,10 @@ __device__ __forceinline__ void pack_tile(const RowsParams& p, TileIndex ti,
   constexpr int NU = (16 * BITS + 31) / 32;
   const int nbytes = (nv * BITS) >> 3;
   const int64_t sym0 = static_cast<int64_t>(tc.half) * p.T + tc.t0;
+  const LanePlanes<ONEBLK> planes = lane_planes<ONEBLK>(p, tc, desc);
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
-    const int64_t d = desc[tc.slot * 16 + k];
+    const int64_t d = planes.get(k);
     if (d < 0) continue;
     const int64_t P = d + p.bit_bias + sym0 * BITS;  // byte aligned unless kRowsBits
     uint32_t u[NU > 4 ? NU : 4];
@@ -1547,31 +1669,29 @@ template <int BITS, int MODE, bool ONEBLK>
 __global__ __launch_bounds__(kRowsThreads) void rows_pack_kernel(RowsParams p) {
   __shared__ int64_t desc[kTilePlanes];
   for (int64_t tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
-    const TileIndex ti = split_tile(p, tile);
-    load_descriptors(p, ti, desc);
+    const bool in_place8 = BITS == 8 && MODE == kRowsBytes;
+    const TileIndex ti =
+        split_tile(p, in_place8 ? xcd_run_order(tile, p.ntiles, p.xcd_run) : tile);
+    if (!ONEBLK || p.planes) load_descriptors(p, ti, desc);
     pack_tile<BITS, MODE, ONEBLK>(p, ti, desc);
   }
 }
 
-// The 8-bit pack off 128-byte lines (kRowsStaged8), for workgroups of WAVES
-// waves (p.waves == WAVES): LDS in proportion, so that the smaller workgroups
-// of short launches still share a CU.
-// The staged pack's regions share their
-// first and last stream lines with the token-neighbouring tiles, so those
-// lines are written in two parts.  Dealing runs of kStagedXcdRun consecutive
+// The 8-bit pack off 128-byte lines (kRowsStaged8), 16-wave workgroups, at 8 or more
+// waves per CU (set_pack_grid), where the block-table walk is the faster row order.
+// Without OWN the regions share their first and last stream lines with the
+// token-neighbouring tiles, so those lines are written in two parts.  Dealing runs of kStagedXcdRun consecutive
 // token tiles to one XCD (workgroups b, b + 8, ... of a group of 8 runs) puts
 // both parts of most shared lines into one L2 at about the same time.  Pack
 // GB/s, runs of 1 / 4 / 16 / 32 / 64 tiles: 32753 tokens 3894 / 4247 / 4448 /
-// 4411 / 4470; 49217 tokens 3340 / - / 3638 / 3622 / 3496; launches with
-// fewer tiles than a group (8199, 4100 tokens) unchanged.
+// 4411 / 4470; 49217 tokens 3340 / - / 3638 / 3622 / 3496.
 constexpr int kStagedXcdRun = 16;
 constexpr int kStagedNtTiles = 4;
 
-template <int WAVES, bool ONEBLK, bool OWN = false>
-__global__ __launch_bounds__(WAVES * 64) void rows_pack_staged8_kernel(RowsParams p) {
-  static_assert(!OWN || (WAVES == 16 && !ONEBLK), "single-owner tiles: 16 waves, row walk");
+template <bool OWN>
+__global__ __launch_bounds__(kRowsThreads) void rows_pack_staged8_kernel(RowsParams p) {
   __shared__ int64_t desc[kRowsWq * kWavePlanes];
-  __shared__ __align__(16) uint8_t stage[2 * stage_round_bytes(WAVES)];
+  __shared__ __align__(16) uint8_t stage[2 * kStageRoundBytes];
   for (int64_t t = blockIdx.x; t < p.ntiles; t += gridDim.x) {
     const int64_t tile = xcd_run_order(t, p.ntiles, kStagedXcdRun);
     const TileIndex ti = split_tile(p, tile);
@@ -1579,7 +1699,7 @@ __global__ __launch_bounds__(WAVES * 64) void rows_pack_staged8_kernel(RowsParam
     if constexpr (OWN)
       pack_tile_owned(p, ti, desc, stage);
     else
-      pack_tile_staged8<WAVES, ONEBLK>(p, ti, desc, stage);
+      pack_tile_staged8(p, ti, desc, stage);
   }
 }
 
@@ -1826,14 +1946,41 @@ int device_cu_count() {
   return n;
 }
 
+// The kernels' divisors; the token tile's is set per launch (by_st).
+void set_divisors(RowsParams& p) {
+  p.by_qt = fast_div(p.nqt);
+  p.by_h = fast_div(p.H);
+  const int64_t most = int64_t(1) << 31;
+  p.by_bs = p.bs < most && p.row_tokens < most ? fast_div(p.bs) : FastDiv{};
+}
+
+// Waves of a tile in a launch of fewer than two 4-wave tiles per CU, `units` wave tiles
+// of work: 2 or 1 where they lower the most waves a CU gets (tiles per CU rounded up,
+// less 5% of a CU, times waves per tile) by enough to pay for the shorter runs.  Restore
+// of Llama-3-8B geometry, us with 4 / 2 / 1 waves: 1024 tokens 5.99 / 4.56 / 3.93, 2176
+// 6.24 / 6.74 / 5.87, 4096 7.27 / 8.54 / 7.54, 4104 9.20 / 10.32 / 10.23, 5001 14.3 /
+// 14.7 / 11.6, 6144 14.4 / 13.2 / 13.0, 7168 14.0 / 16.1 / 14.5; pack 1024 tokens 6.48 /
+// 5.63 / 5.20, 4096 8.21 / 8.14 / 8.87, 5120 12.5 / 9.9 / 9.4, 7168 13.1 / 13.3 / 12.0.
+int short_tile_waves(double units, bool pack) {
+  const double cus = device_cu_count();
+  auto load = [&](int waves) {
+    return std::max(1.0, std::ceil((units - 0.05 * cus) / (cus * waves))) * waves;
+  };
+  int best = 4;
+  for (int waves = 2; waves >= 1; waves /= 2)
+    if (load(waves) <= (pack ? 0.9 : 0.85) * load(best)) best = waves;
+  return best;
+}
+
 // Grid of the rows kernels.  When heads are contiguous inside a row
 // (head_pitch == C) and the plane table is indexed h * C + c, the heads are
 // folded into one row of H * C channels so a workgroup can span them.  The
-// workgroup is the largest of 16, 8 or 4 waves that still gives at least two
+// workgroup is the largest of 16, 8 or 4 waves (or, in short launches, 2 or 1:
+// short_tile_waves) that still gives at least two
 // workgroups per CU over `nhalf` halves of `tile_tokens_total` tokens.
 void set_grid_dims(RowsParams& p, int64_t H, int64_t C, int64_t tile_tokens_total,
                    int64_t nhalf, int wq_max = kRowsWq, int seg_tokens = kSegTokens,
-                   int max_waves = kRowsMaxWaves, int64_t want_tiles = 0) {
+                   int max_waves = kRowsMaxWaves, int64_t want_tiles = 0, bool pack = false) {
   if (H > 1 && p.head_pitch == C) {
     C *= H;
     H = 1;
@@ -1861,19 +2008,11 @@ void set_grid_dims(RowsParams& p, int64_t H, int64_t C, int64_t tile_tokens_tota
   int waves = max_waves;
   int64_t tiles = shape(waves);
   while (tiles < want && waves > 4) tiles = shape(waves /= 2);
-  // Short of `want` at 4 waves: 2-wave tiles when they lower the most work a
-  // CU gets (tiles per CU rounded up, times waves per tile).  Restore / pack
-  // of Llama-3-8B geometry, us / GB/s: 2048 tokens 6.87 -> 5.61 / 2515 ->
-  // 2793, 6144 tokens 14.1 -> 12.0 / 3650 -> 4644; where it is a tie (4096,
-  // 7168 tokens) 2-wave tiles ran up to 15% slower.  Not for the staged pack
-  // (wq_max 1), whose workgroups hold LDS rounds for 4 waves or more.
+  // Not for the staged pack (wq_max 1), whose workgroups hold LDS rounds for 4 waves or
+  // more.
   if (tiles < want && waves == 4 && wq_max != 1) {
-    const int64_t load4 = (tiles + cus - 1) / cus * 4;
-    const int64_t tiles2 = shape(2);
-    if ((tiles2 + cus - 1) / cus * 2 < load4)
-      tiles = tiles2;
-    else
-      tiles = shape(4);
+    const double units = static_cast<double>(nhalf * H * nqg) * segs / kLaneSegs;
+    tiles = shape(short_tile_waves(units, pack));
   }
   const int64_t segs_per_wg = static_cast<int64_t>(p.ws) * kLaneSegs;
   p.partial_last = p.nst > 1 && segs % segs_per_wg != 0;
@@ -1915,13 +2054,12 @@ void set_batch_grid(RowsBatch& b, int64_t H, int64_t C) {
   int waves = kRowsMaxWaves;
   int64_t tiles = shape(waves);
   while (tiles < want && waves > 4) tiles = shape(waves /= 2);
-  // short of `want` at 4 waves: 2-wave tiles when they lower the most work a
-  // CU gets, as set_grid_dims does for one request
-  if (tiles < want && waves == 4) {
-    const int64_t cus = device_cu_count();
-    const int64_t load4 = (tiles + cus - 1) / cus * 4;
-    const int64_t tiles2 = shape(2);
-    if ((tiles2 + cus - 1) / cus * 2 >= load4) shape(4);
+  if (tiles < want && waves == 4) {  // as set_grid_dims does for one request
+    double units = 0;
+    for (int r = 0; r < b.nreq; ++r)
+      units += static_cast<double>(2 * H * nqg) *
+               ((b.req[r].row_tokens - b.req[r].token0 + kSegTokens - 1) / kSegTokens) / kLaneSegs;
+    shape(short_tile_waves(units, false));
   }
   const int64_t per = 2 * H * static_cast<int64_t>(p.nqt);  // tiles per token tile
   const int64_t tile_tokens = static_cast<int64_t>(p.ws) * kLaneSegs * kSegTokens;
@@ -1931,7 +2069,9 @@ void set_batch_grid(RowsBatch& b, int64_t H, int64_t C) {
     b.req[r].nst = static_cast<int32_t>(nst_of(n));
     b.req[r].partial = n % tile_tokens != 0 ? 1 : 0;
     b.req[r].tile0 = tile0;
-    tile0 += per * (b.req[r].nst - b.req[r].partial);
+    const int full = b.req[r].nst - b.req[r].partial;
+    b.req[r].by_st = fast_div(full > 0 ? full : 1);
+    tile0 += per * full;
   }
   b.nfull = tile0;
   for (int r = 0; r < b.nreq; ++r) {
@@ -1939,6 +2079,10 @@ void set_batch_grid(RowsBatch& b, int64_t H, int64_t C) {
     tile0 += per * b.req[r].partial;
   }
   p.ntiles = tile0;
+  set_divisors(p);
+  const int64_t most = int64_t(1) << 31;
+  for (int r = 0; r < b.nreq; ++r)
+    if (b.req[r].row_tokens >= most) p.by_bs = FastDiv{};
 }
 
 // Average waves per CU over a launch of `ntiles` workgroups of `waves` waves,
@@ -1949,9 +2093,8 @@ double waves_per_cu(int64_t ntiles, int waves) {
 }
 
 // Row order of the whole-tile row kernels by launch size (waves per CU).
-// One-block rows (for_rows16) for restores and staged packs up to 6 waves per
-// CU (4096 tokens of Llama-3-8B: 9.6 -> 8.0 us; 8192 tokens: 14.0 -> 14.6, so
-// not above), for the other packs up to 12 (4096 tokens: 2.07 -> 4.03 TB/s;
+// One-block rows (for_rows16) for restores up to 6 waves per CU (4096 tokens of
+// Llama-3-8B: 9.6 -> 8.0 us; 8192 tokens: 14.0 -> 14.6, so not above), for packs up to 12 (4096 tokens: 2.07 -> 4.03 TB/s;
 // 12288: 4.50 -> 4.74; 16384 tokens at 16: 5.07 -> 4.83).  Serial plane loads
 // (load_planes16) for b = 7, 8 shift restores above 12 waves per CU.
 constexpr double kOneBlockWaves = 6;
@@ -2100,37 +2243,54 @@ int pack_mode(const PlanInfo& info, const RowsParams& p, int64_t T) {
 // 256 x 1024 tiles).
 constexpr int kStagedWq = 1;
 
-// Workgroup grid of a pack in `mode`.  The staged pack takes the largest
-// workgroups that still give half a tile per CU (the rows kernels want two):
-// its LDS rounds and barriers favour fewer, larger tiles.  GB/s with 4-, 8-
-// and 16-wave workgroups: 4100 tokens 1550 / 1649 / 1375, 8200 tokens 2320 /
-// 2315 / 2482, 15000 tokens 3235 / 3565 / 3824; at 2053 tokens 4-wave tiles
-// stay fastest (955 against 901 / 699).
-void set_pack_grid(RowsParams& p, int mode, int64_t H, int64_t C, int64_t T, int64_t nhalf) {
+// Workgroup grid of a pack in `mode`; returns the mode, kRowsBytes where an 8-bit pack
+// off 128-byte lines is better written run by run, each 16-byte run in one store at its
+// byte, than staged.  The staged pack holds one 16-wave tile per CU at a time and has
+// two partial chunks per region and plane to write, 24-29 us for each round of tiles
+// however full (and as much for the smaller tiles of a short launch); runs in place cost
+// by the byte.  So runs go in place where there is less than half a tile per CU, where
+// the rounds would be at most 69% full, and, if runs start on dwords, beyond two rounds.
+// us per layer of Llama-3-8B geometry, staged / in place: 777 tokens 16.4 / 6.7, 4104
+// 19.4 / 12.7, 8201 23.9 / 22.4, 11008 (67%) 21.4 / 21.4, 12001 (73%) 25.7 / 26.2, 18000
+// (55%) 44.0 / 39.9, 24001 (73%) 46.8 / 50.8, 30000 (92%) 50.5 / 56.7, 32784 (67%) 67.9 /
+// 60.9, 49217 (75%, bytes) 95.4 / 97.8, 57360 (88%) 107.6 / 100.0.
+constexpr double kStagedFull = 0.69;
+
+int set_pack_grid(RowsParams& p, const PlanInfo& info, int mode, int64_t H, int64_t C, int64_t T,
+                  int64_t nhalf) {
   p.own_lines = 0;
+  p.xcd_run = 1;
   if (mode == kRowsStaged8) {
+    const int64_t cus = device_cu_count();
     set_grid_dims(p, H, C, T, nhalf, kStagedWq, kSegTokens, kRowsMaxWaves,
-                  std::max<int64_t>(1, device_cu_count() / 2));
-    // 16-wave tiles write each stream line from one tile (kOwnTokens per
-    // tile) when that takes no more rounds of tiles per CU (one 16-wave tile
-    // per CU at a time): the smaller tiles are more of them, and a further
-    // round cost more than single ownership saves.  µs per layer, two-part
-    // lines -> single owner: 49217 tokens 111.0 -> 103.4 (4 rounds either
-    // way); 32753 tokens 62.9 -> 73.3 and 16383 tokens 30.5 -> 46.5 (2 -> 3
-    // and 1 -> 2 rounds: not taken).
-    if (p.waves == 16 && p.wq == 1 && T >= 128 && nhalf == 2) {
+                  std::max<int64_t>(1, cus / 2));
+    const int64_t per_st = nhalf * p.H * static_cast<int64_t>(p.nqt);
+    const int64_t rounds = (per_st * p.nst + cus - 1) / cus;
+    const double full = static_cast<double>(per_st) * T /
+                        (kRowsMaxWaves * kLaneSegs * kSegTokens) / (rounds * cus);
+    const bool dwords = T % 4 == 0 && info.planes_dword && p.bit_bias == 0;
+    if (p.waves < kRowsMaxWaves || p.wq != 1 || full <= kStagedFull || (dwords && rounds > 2)) {
+      mode = kRowsBytes;
+      // up to two rounds' work, runs of token tiles on one XCD, which share lines: 4104
+      // tokens 13.1 -> 12.7 us, 9001 25.3 -> 23.3; above, 32784 60.9 -> 63.9
+      if (rounds <= 2) p.xcd_run = kStagedXcdRun;
+    } else if (T >= 128 && nhalf == 2) {
+      // Tiles write each stream line from one tile (kOwnTokens per tile) when that takes
+      // no more rounds of tiles per CU: the smaller tiles are more of them, and a further
+      // round cost more than single ownership saves.  µs per layer, two-part lines ->
+      // single owner: 49217 tokens 111.0 -> 103.4 (4 rounds either way); 32753 tokens
+      // 62.9 -> 73.3 and 16383 tokens 30.5 -> 46.5 (2 -> 3 and 1 -> 2 rounds: not taken).
       const int64_t nst_own = (T + kOwnTokens - 1) / kOwnTokens;
-      const int64_t per_st = nhalf * p.H * static_cast<int64_t>(p.nqt);
-      const int64_t cus = device_cu_count();
-      if ((per_st * nst_own + cus - 1) / cus <= (per_st * p.nst + cus - 1) / cus) {
+      if ((per_st * nst_own + cus - 1) / cus <= rounds) {
         p.own_lines = 1;
         p.nst = static_cast<int32_t>(nst_own);
         p.partial_last = 0;
       }
     }
-  } else {
-    set_grid_dims(p, H, C, T, nhalf);
   }
+  if (mode != kRowsStaged8)
+    set_grid_dims(p, H, C, T, nhalf, kRowsWq, kSegTokens, kRowsMaxWaves, 0, true);
+  return mode;
 }
 
 template <int BITS, int MODE>
@@ -2155,21 +2315,6 @@ void launch_pack_tiles(dim3 grid, dim3 block, hipStream_t stream, const RowsPara
     hipLaunchKernelGGL((rows_pack_kernel<BITS, MODE, true>), grid, block, 0, stream, p);
   else
     hipLaunchKernelGGL((rows_pack_kernel<BITS, MODE, false>), grid, block, 0, stream, p);
-}
-
-template <int WAVES>
-void launch_staged_tiles(dim3 grid, dim3 block, hipStream_t stream, const RowsParams& p,
-                         bool oneblk) {
-  if constexpr (WAVES == 16) {
-    if (p.own_lines) {  // the row walk whatever `oneblk` says (pack_tile_owned)
-      hipLaunchKernelGGL((rows_pack_staged8_kernel<16, false, true>), grid, block, 0, stream, p);
-      return;
-    }
-  }
-  if (oneblk)
-    hipLaunchKernelGGL((rows_pack_staged8_kernel<WAVES, true>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((rows_pack_staged8_kernel<WAVES, false>), grid, block, 0, stream, p);
 }
 
 template <int BITS>
@@ -2237,6 +2382,10 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
   // partial token tiles last: restore 32784 tokens 64.0 -> 61.4 us, 49216
   // tokens 96.8 -> 94.8 us; the pack ran 2-5% slower that way
   if (pack) p.partial_last = 0;
+  const int full = p.nst - (p.partial_last ? 1 : 0);
+  p.nfull = static_cast<uint32_t>(p.ntiles / p.nst * full);
+  p.by_st = fast_div(full);
+  set_divisors(p);
   if (!pack && mode != kRowsWide && mode != kRowsWideCached && p.waves > kRowsSplitWaves &&
       p.ntiles >= kRowsSplitTiles * static_cast<int64_t>(device_cu_count()))
     return launch_rows_split(p, bits, mode, stream);
@@ -2247,7 +2396,7 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
   const double wpc = waves_per_cu(p.ntiles, p.waves);
   const bool staged = mode == kRowsStaged8;
   const bool oneblk =
-      one_block_rows(p) && wpc <= (pack && !staged ? kOneBlockPackWaves : kOneBlockWaves);
+      one_block_rows(p) && wpc <= (pack ? kOneBlockPackWaves : kOneBlockWaves);
   const bool serial = wpc > kSerialLoadWaves;
   if (mode == kRowsWide || mode == kRowsWideCached) {
     if (pack || p.waves > kWideMaxWaves)
@@ -2275,8 +2424,12 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
       launch_unpack_tiles<8, kRowsAligned16>(grid, block, stream, p, oneblk, serial);
     return check_launch(pack ? "rows_pack_kernel" : "rows_unpack_kernel");
   }
-  if (pack && bits == 8 && !staged)  // pack_mode: aligned16 or staged
-    return fail(ORIGAMI_ERR_INVALID, "8-bit rows pack modes are aligned16 and staged");
+  if (pack && bits == 8 && mode == kRowsBytes) {
+    launch_pack_tiles<8, kRowsBytes>(grid, block, stream, p, oneblk);
+    return check_launch("rows_pack_kernel");
+  }
+  if (pack && bits == 8 && !staged)  // pack_mode
+    return fail(ORIGAMI_ERR_INVALID, "8-bit rows pack modes are aligned16, bytes and staged");
   if (bits == 8 && mode == kRowsAligned16Cached) {
     launch_unpack_tiles<8, kRowsAligned16Cached>(grid, block, stream, p, oneblk, serial);
     return check_launch("rows_unpack_kernel");
@@ -2290,14 +2443,12 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
     // 3638 / 3645 -> 3766 / 3776; 65521 tokens (4 tiles per CU): 4203 / 4201
     // -> 4135 / 4119.
     p.nt_stores = p.ntiles < kStagedNtTiles * static_cast<int64_t>(device_cu_count());
-    if (p.waves == 16)
-      launch_staged_tiles<16>(grid, block, stream, p, oneblk);
-    else if (p.waves == 8)
-      launch_staged_tiles<8>(grid, block, stream, p, oneblk);
-    else if (p.waves == 4)
-      launch_staged_tiles<4>(grid, block, stream, p, oneblk);
+    if (p.waves != kRowsMaxWaves || p.wq != 1)
+      return fail(ORIGAMI_ERR_INVALID, "staged pack workgroups have 16 waves");
+    if (p.own_lines)
+      hipLaunchKernelGGL((rows_pack_staged8_kernel<true>), grid, block, 0, stream, p);
     else
-      return fail(ORIGAMI_ERR_INVALID, "staged pack workgroups have 4, 8 or 16 waves");
+      hipLaunchKernelGGL((rows_pack_staged8_kernel<false>), grid, block, 0, stream, p);
     return check_launch("rows_pack_staged8_kernel");
   }
   if (mode == kRowsBits && (!pack || bits >= 8))
@@ -2324,7 +2475,7 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
     ORIGAMI_ROWS_CASE(5)
     ORIGAMI_ROWS_CASE(6)
     ORIGAMI_ROWS_CASE(7)
-    case 8:  // restore only: the 8-bit pack is aligned16 or staged
+    case 8:  // restore only: the 8-bit pack was launched above
       if (window)
         launch_unpack_tiles<8, kRowsWindow>(grid, block, stream, p, oneblk, serial);
       else
@@ -2780,8 +2931,7 @@ int origami_pack_canonical_storage_chunks(
     p.row_pitch = st.token;
     p.head_pitch = st.head;
     p.bs = T;
-    const int mode = pack_mode(plan->info, p, T);
-    set_pack_grid(p, mode, H, C, T, 1);
+    const int mode = set_pack_grid(p, plan->info, pack_mode(plan->info, p, T), H, C, T, 1);
     if (int rc2 = clear_bits_stream(mode, flat_chunks, chunk_offsets, num_chunks, stream))
       return rc2;
     return launch_rows(true, p, 1, plan->info.bits, mode, stream);
@@ -3063,8 +3213,8 @@ int origami_pack_canonical_from_kv_cache(
   p.bs = block_size;
   p.blk_stride = blk_stride;
   p.half_stride = half_stride;
-  const int mode = pack_mode(plan->info, p, tokens);
-  set_pack_grid(p, mode, num_heads, head_bytes, tokens, 2);
+  const int mode = set_pack_grid(p, plan->info, pack_mode(plan->info, p, tokens), num_heads,
+                                 head_bytes, tokens, 2);
   if (int rc2 = clear_bits_stream(mode, flat_chunks, chunk_offsets, num_chunks, stream))
     return rc2;
   return launch_rows(true, p, 2, plan->info.bits, mode, stream);
