@@ -12,7 +12,7 @@
 //
 // HBM bounds both: 4 bytes read and b / 4 bytes written per (K, V) pair of 16-bit
 // values.  16384 tokens of 8 heads x 128, bf16, with the copy of the payload into its
-// stored chunks: CacheGen 573 -> 26.7 us, KIVI (2 bits) 1025 -> 33.3 us.
+// stored chunks: CacheGen 573 -> 26.7 us, KIVI (2 bits) 1025 -> 30.1 us.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -246,19 +246,16 @@ struct KiviQuantParams {
 constexpr int kQTokens = 16;  // tokens of a lane
 
 // Two float16 values per register: the ranges are taken on pairs.
-__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+// The least and greatest of three, NaN if one is a NaN (gfx950's IEEE 754-2019 minimum
+// and maximum).
+__device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
-  asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
-__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
+__device__ __forceinline__ uint32_t pk_max3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
-  asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
-}
-__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
-  uint32_t r;
-  asm("v_pk_max_u16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 __device__ __forceinline__ float low_half(uint32_t v) {
@@ -273,12 +270,14 @@ struct Group {
   float zero, scale, inv;
 };
 
-// `range` holds the minimum (low) and the negated maximum (high).
-__device__ __forceinline__ Group make_group(uint32_t range, bool nan, float inv_levels) {
+// `range` holds the minimum (low) and the negated maximum (high); one is a NaN if the
+// other is.
+__device__ __forceinline__ Group make_group(uint32_t range, float inv_levels) {
   const float tiny = 1.17549435e-38f;  // the least normal binary32
   Group g;
-  g.zero = nan ? __builtin_nanf("") : low_half(range);
-  const float top = nan ? __builtin_nanf("") : high_half(range ^ 0x80000000u);
+  const float low = low_half(range);
+  g.zero = low == low ? low : __builtin_nanf("");
+  const float top = low == low ? high_half(range ^ 0x80000000u) : __builtin_nanf("");
   const float s = __fmul_rn(__fsub_rn(top, g.zero), inv_levels);
   g.scale = s < tiny ? tiny : s;
   g.inv = __fdiv_rn(1.0f, g.scale);
@@ -290,12 +289,31 @@ __device__ __forceinline__ Group make_group(uint32_t range, bool nan, float inv_
 // (Markstein's division; nothing underflows here, as a scale is the least normal number
 // where the group has one value, and at least 2^-32 elsewhere).  An infinite or NaN
 // scale gives a NaN, whose symbol is 0 like that of the quotient.
-__device__ __forceinline__ float kivi_symbol(float x, const Group& g) {
-  const float d = __fsub_rn(x, g.zero);
+// x is the low or high half of `pair`: one v_fma_mix converts it and takes off the zero
+// point (x * 1 - zero, rounded once, as the subtraction).
+template <bool HIGH>
+__device__ __forceinline__ float kivi_symbol(uint32_t pair, const Group& g) {
+  float d;
+  if constexpr (HIGH)
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(d) : "v"(pair), "v"(g.zero));
+  else
+    asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(pair), "v"(g.zero));
   const float q0 = __fmul_rn(d, g.inv);
   const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, g.scale, d), g.inv, q0);
   const float q2 = __builtin_fmaf(__builtin_fmaf(-q1, g.scale, d), g.inv, q1);
   return __builtin_rintf(fmaxf(q2, 0.0f));
+}
+
+// Eight values as float16 at any even address.
+__device__ __forceinline__ void store_halves(uint16_t* dst, const float (&v)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const f32x2 pair = {v[2 * k], v[2 * k + 1]};
+    w[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, f16x2));
+  }
+  *reinterpret_cast<u32x4u*>(dst) = u32x4u{w[0], w[1], w[2], w[3]};
 }
 
 // A lane's run of one plane: 16 symbols of W bits, gathered as exact binary32 sums of
@@ -361,7 +379,10 @@ __device__ __forceinline__ void each(F&& f) {
 // channel load the last one again, which changes no range of a group they share.
 // With the loads in flight the arithmetic bounds it: ranges on pairs, a branch-free
 // division and symbols gathered by fused multiply-adds took the save of 16384 tokens
-// from 61.0 us (scalar ranges, a branch per quotient, shifts) to 33.3.
+// from 61.0 us (scalar ranges, a branch per quotient, shifts) to 33.3; ranges by the
+// three-operand minimum and maximum, which carry NaNs, the subtraction of the zero point
+// folded into the conversion and one address per lane to 30.1.  A cap of 96 registers
+// for five waves per SIMD spills (58 us).
 template <int HALF, int DT, int W, bool BYTES>
 __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uint32_t tile) {
   constexpr int CL = HALF == 0 ? 8 : 16, TL = 64 / CL;  // lanes along channels, tokens
@@ -383,15 +404,23 @@ __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uin
     uint32_t t = p.sink + bt0 < last ? p.sink + bt0 : last;
     uint32_t blk = t / p.s.block_tokens, off = t - blk * p.s.block_tokens;
     Eight<DT> x[kQTokens];
+    if (__all(t + kQTokens - 1 <= last && off + kQTokens <= p.s.block_tokens)) {
+      // every lane's tokens are rows of one block: one address, a uniform step
+      const int64_t row = static_cast<int64_t>(blk) * p.s.block +
+                          static_cast<int64_t>(off) * p.s.token + col;
 #pragma unroll
-    for (int j = 0; j < kQTokens; ++j) {
-      x[j].load(p.kv, static_cast<int64_t>(blk) * p.s.block +
-                          static_cast<int64_t>(off) * p.s.token + col);
-      if (t < last) {
-        ++t;
-        if (++off == p.s.block_tokens) {
-          off = 0;
-          ++blk;
+      for (int j = 0; j < kQTokens; ++j) x[j].load(p.kv, row + j * p.s.token);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kQTokens; ++j) {
+        x[j].load(p.kv, static_cast<int64_t>(blk) * p.s.block +
+                            static_cast<int64_t>(off) * p.s.token + col);
+        if (t < last) {
+          ++t;
+          if (++off == p.s.block_tokens) {
+            off = 0;
+            ++blk;
+          }
         }
       }
     }
@@ -410,75 +439,74 @@ __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uin
   }
 
   PlaneRun<W> run[8];
-  const uint32_t kAbs = 0x7fff7fffu, kNegHigh = 0x80000000u;
+  const uint32_t kNegHigh = 0x80000000u;
   if constexpr (HALF == 0) {
     const int lanes = p.group / kQTokens;  // token lanes of a group
-    uint32_t range[8], nans = 0;
+    uint32_t range[8];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      uint32_t lo = v[0][k], hi = v[0][k], top = v[0][k] & kAbs;
+      uint32_t lo = v[0][k], hi = v[0][k];
 #pragma unroll
-      for (int j = 1; j < kQTokens; ++j) {
-        lo = pk_min(lo, v[j][k]);
-        hi = pk_max(hi, v[j][k]);
-        top = pk_max_u16(top, v[j][k] & kAbs);
+      for (int j = 1; j < kQTokens; j += 2) {
+        const uint32_t a = v[j][k], b = v[j + 1 < kQTokens ? j + 1 : j][k];
+        lo = pk_min3(lo, a, b);
+        hi = pk_max3(hi, a, b);
       }
       range[2 * k] = __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ kNegHigh;
       range[2 * k + 1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ kNegHigh;
-      nans |= ((top & 0xffffu) > 0x7c00u ? 1u : 0u) << (2 * k);
-      nans |= (top > 0x7c00ffffu ? 2u : 0u) << (2 * k);
     }
-    for (int m = 1; m < lanes; m <<= 1) {
-      nans |= __shfl_xor(nans, m * CL);
+    for (int m = 1; m < lanes; m <<= 1)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) range[i] = pk_min(range[i], __shfl_xor(range[i], m * CL));
-    }
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t o = __shfl_xor(range[i], m * CL);
+        range[i] = pk_min3(range[i], o, o);
+      }
     const int64_t meta = static_cast<int64_t>(bt0 / p.group) * p.C + c0;
     const bool lead = nv > 0 && bt0 % p.group == 0;
+    float scales[8], zeros[8];
     each<8>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      const Group g = make_group(range[i], (nans >> i) & 1, p.inv_levels);
-      if (lead) {
-        p.scale[0][meta + i] = half_bits(g.scale);
-        p.zero[0][meta + i] = half_bits(g.zero);
-      }
+      const Group g = make_group(range[i], p.inv_levels);
+      scales[i] = g.scale;
+      zeros[i] = g.zero;
       each<kQTokens>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        run[i].template put<j>(
-            kivi_symbol(i & 1 ? high_half(v[j][i >> 1]) : low_half(v[j][i >> 1]), g));
+        run[i].template put<j>(kivi_symbol<(i & 1) != 0>(v[j][i >> 1], g));
       });
     });
+    if (lead) {
+      store_halves(p.scale[0] + meta, scales);
+      store_halves(p.zero[0] + meta, zeros);
+    }
   } else {
     const int lanes = p.group / 8;  // channel lanes of a group
-    uint32_t range[kQTokens], nans = 0;
+    uint32_t range[kQTokens];
 #pragma unroll
     for (int j = 0; j < kQTokens; ++j) {
-      const uint32_t lo = pk_min(pk_min(v[j][0], v[j][1]), pk_min(v[j][2], v[j][3]));
-      const uint32_t hi = pk_max(pk_max(v[j][0], v[j][1]), pk_max(v[j][2], v[j][3]));
-      const uint32_t top = pk_max_u16(pk_max_u16(v[j][0] & kAbs, v[j][1] & kAbs),
-                                      pk_max_u16(v[j][2] & kAbs, v[j][3] & kAbs));
-      range[j] = pk_min(__builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ kNegHigh,
-                        __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ kNegHigh);
-      nans |= ((top & 0xffffu) > 0x7c00u || top > 0x7c00ffffu ? 1u : 0u) << j;
+      const uint32_t lo = pk_min3(pk_min3(v[j][0], v[j][1], v[j][2]), v[j][3], v[j][3]);
+      const uint32_t hi = pk_max3(pk_max3(v[j][0], v[j][1], v[j][2]), v[j][3], v[j][3]);
+      const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ kNegHigh;
+      const uint32_t b = __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ kNegHigh;
+      range[j] = pk_min3(a, b, b);
     }
-    for (int m = 1; m < lanes; m <<= 1) {
-      nans |= __shfl_xor(nans, m);
+    for (int m = 1; m < lanes; m <<= 1)
 #pragma unroll
-      for (int j = 0; j < kQTokens; ++j) range[j] = pk_min(range[j], __shfl_xor(range[j], m));
-    }
+      for (int j = 0; j < kQTokens; ++j) {
+        const uint32_t o = __shfl_xor(range[j], m);
+        range[j] = pk_min3(range[j], o, o);
+      }
     const bool lead = chan_ok && c0 % p.group == 0;
     const int64_t meta = static_cast<int64_t>(bt0) * p.vgroups + c0 / p.group;
     each<kQTokens>([&](auto jc) {
       constexpr int j = decltype(jc)::value;
-      const Group g = make_group(range[j], (nans >> j) & 1, p.inv_levels);
+      const Group g = make_group(range[j], p.inv_levels);
       if (lead && j < nv) {
         p.scale[1][meta + static_cast<int64_t>(j) * p.vgroups] = half_bits(g.scale);
         p.zero[1][meta + static_cast<int64_t>(j) * p.vgroups] = half_bits(g.zero);
       }
       each<8>([&](auto ic) {
         constexpr int i = decltype(ic)::value;
-        run[i].template put<j>(
-            kivi_symbol(i & 1 ? high_half(v[j][i >> 1]) : low_half(v[j][i >> 1]), g));
+        run[i].template put<j>(kivi_symbol<(i & 1) != 0>(v[j][i >> 1], g));
       });
     });
   }

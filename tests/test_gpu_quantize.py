@@ -95,6 +95,7 @@ def test_unusual_values(cuda_device, dtype, monkeypatch):
     flat[:, 80] = torch.finfo(torch.float16).tiny / 2
     flat[:, 81] = 1e-7
     flat[:, 82, 3] = 6e4
+    flat[:, 96:112] *= 1e-6  # float16 subnormals
     _check_cachegen(kv, {}, 4, monkeypatch)
     for bits in (2, 8):
         _check_kivi(kv, {"bits": bits, "group_size": 64, "sink_tokens": 0}, monkeypatch)
