@@ -166,24 +166,27 @@ __device__ __forceinline__ float cachegen_level(int s, float center) {
 // CacheGen -> paged KV cache
 // ---------------------------------------------------------------------------
 
-struct CacheGenCacheParams {
+struct CacheGenHalf {
   ByteStream s;
-  const void* maxv;       // per-token maxima of this half
+  const void* maxv;       // per-token maxima
+  float center;
+  int32_t bits;
+};
+
+struct CacheGenCacheParams {
+  CacheGenHalf half[2];   // blockIdx.y: keys, values
   uint16_t* cache;
   const int64_t* block_ids;
   int64_t num_blocks, block_count, bs;
-  int64_t blk_stride, half_stride, half;  // in rows of C elements
+  int64_t blk_stride, half_stride;  // in rows of C elements
   int64_t tokens;
   int64_t C;              // heads * head_dim, a multiple of 8
-  float center;
 };
 
 template <int BITS, bool BF16, bool MAX_HALF>
-__global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCacheParams p) {
-  __shared__ float lut[1 << BITS];
-  for (int i = threadIdx.x; i < (1 << BITS); i += kCgThreads) lut[i] = cachegen_level(i, p.center);
-  __syncthreads();
-
+__device__ __forceinline__ void cachegen_cache_blocks(const CacheGenCacheParams& p,
+                                                      const float* lut) {
+  const CacheGenHalf& q = p.half[blockIdx.y];
   const int32_t G = static_cast<int32_t>(p.C >> 3);  // groups per token row
   const int32_t t_step = kCgThreads / G, c_step = kCgThreads % G;
   const int32_t tt0 = static_cast<int32_t>(threadIdx.x) / G;
@@ -197,7 +200,7 @@ __global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCach
     int64_t nt64 = p.tokens - t0;
     if (nt64 <= 0) continue;
     const int32_t nt = static_cast<int32_t>(nt64 < p.bs ? nt64 : p.bs);
-    uint16_t* dst = p.cache + (pid * p.blk_stride + p.half * p.half_stride) * p.C;
+    uint16_t* dst = p.cache + (pid * p.blk_stride + blockIdx.y * p.half_stride) * p.C;
     const int64_t g0 = t0 * G;  // first 8-symbol group of the block's rows
     int32_t tt = tt0, cg = cg0;
     // kCgBatch groups at a time: every group's dwords and maximum are
@@ -217,16 +220,16 @@ __global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCach
         w[j][0] = w[j][1] = w[j][2] = 0;
         mraw[j] = 0;
         if (tt < nt) {
-          const int64_t o = p.s.bias + (g0 + static_cast<int64_t>(tt) * G + cg) * BITS;
+          const int64_t o = q.s.bias + (g0 + static_cast<int64_t>(tt) * G + cg) * BITS;
           bo[j] = o;
           const int64_t k0 = o >> 2;
 #pragma unroll
           for (int i = 0; i < NW; ++i)
-            if ((k0 + i) * 4 < p.s.bytes) w[j][i] = p.s.base[k0 + i];
+            if ((k0 + i) * 4 < q.s.bytes) w[j][i] = q.s.base[k0 + i];
           if constexpr (MAX_HALF)
-            mraw[j] = static_cast<const uint16_t*>(p.maxv)[t0 + tt];
+            mraw[j] = static_cast<const uint16_t*>(q.maxv)[t0 + tt];
           else
-            mraw[j] = static_cast<const uint32_t*>(p.maxv)[t0 + tt];
+            mraw[j] = static_cast<const uint32_t*>(q.maxv)[t0 + tt];
         }
         cg += c_step;
         tt += t_step;
@@ -244,7 +247,7 @@ __global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCach
         const uint32_t hi = NW > 2 ? __builtin_amdgcn_alignbyte(w[j][2], w[j][1], sh)
                                    : (w[j][1] >> (8 * sh));
         uint64_t x64 = (static_cast<uint64_t>(hi) << 32) | lo;
-        const int64_t avail = p.s.bytes - bo[j];
+        const int64_t avail = q.s.bytes - bo[j];
         if (avail < BITS) x64 = avail <= 0 ? 0 : (x64 & ((uint64_t(1) << (8 * avail)) - 1));
         float m;
         if constexpr (MAX_HALF)
@@ -263,6 +266,28 @@ __global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCach
             x, reinterpret_cast<u32x4*>(dst + static_cast<int64_t>(bt[j]) * p.C + bc[j] * 8));
       }
     }
+  }
+}
+
+// Both halves in one launch, each with the shifts of its width.  A launch per half left
+// the second to wait for the first's last blocks: a 32768-token Llama-3-8B layer 29.3 us
+// in two launches, 26.7 in one.
+template <bool BF16, bool MAX_HALF>
+__global__ __launch_bounds__(kCgThreads) void cachegen_cache_kernel(CacheGenCacheParams p) {
+  __shared__ float lut[256];
+  const int bits = p.half[blockIdx.y].bits;
+  for (int i = threadIdx.x; i < (1 << bits); i += kCgThreads)
+    lut[i] = cachegen_level(i, p.half[blockIdx.y].center);
+  __syncthreads();
+  switch (bits) {
+    case 1: return cachegen_cache_blocks<1, BF16, MAX_HALF>(p, lut);
+    case 2: return cachegen_cache_blocks<2, BF16, MAX_HALF>(p, lut);
+    case 3: return cachegen_cache_blocks<3, BF16, MAX_HALF>(p, lut);
+    case 4: return cachegen_cache_blocks<4, BF16, MAX_HALF>(p, lut);
+    case 5: return cachegen_cache_blocks<5, BF16, MAX_HALF>(p, lut);
+    case 6: return cachegen_cache_blocks<6, BF16, MAX_HALF>(p, lut);
+    case 7: return cachegen_cache_blocks<7, BF16, MAX_HALF>(p, lut);
+    default: return cachegen_cache_blocks<8, BF16, MAX_HALF>(p, lut);
   }
 }
 
@@ -812,36 +837,17 @@ int check_bits(int64_t bits) {
   return ORIGAMI_OK;
 }
 
-int launch_cachegen_cache(const CacheGenCacheParams& p, int bits, bool bf16, bool max_half,
+int launch_cachegen_cache(const CacheGenCacheParams& p, bool bf16, bool max_half,
                           hipStream_t stream) {
-  const dim3 grid(grid_for(p.block_count, 1, kMaxDqGrid)), block(kCgThreads);
-#define ORIGAMI_CG_CASE(B)                                                                   \
-  case B:                                                                                    \
-    if (bf16) {                                                                              \
-      if (max_half)                                                                          \
-        hipLaunchKernelGGL((cachegen_cache_kernel<B, true, true>), grid, block, 0, stream, p); \
-      else                                                                                   \
-        hipLaunchKernelGGL((cachegen_cache_kernel<B, true, false>), grid, block, 0, stream, p); \
-    } else {                                                                                 \
-      if (max_half)                                                                          \
-        hipLaunchKernelGGL((cachegen_cache_kernel<B, false, true>), grid, block, 0, stream, p); \
-      else                                                                                   \
-        hipLaunchKernelGGL((cachegen_cache_kernel<B, false, false>), grid, block, 0, stream, p); \
-    }                                                                                        \
-    break;
-  switch (bits) {
-    ORIGAMI_CG_CASE(1)
-    ORIGAMI_CG_CASE(2)
-    ORIGAMI_CG_CASE(3)
-    ORIGAMI_CG_CASE(4)
-    ORIGAMI_CG_CASE(5)
-    ORIGAMI_CG_CASE(6)
-    ORIGAMI_CG_CASE(7)
-    ORIGAMI_CG_CASE(8)
-    default:
-      return check_bits(bits);
-  }
-#undef ORIGAMI_CG_CASE
+  const dim3 grid(grid_for(p.block_count, 1, kMaxDqGrid), 2), block(kCgThreads);
+  if (bf16 && max_half)
+    hipLaunchKernelGGL((cachegen_cache_kernel<true, true>), grid, block, 0, stream, p);
+  else if (bf16)
+    hipLaunchKernelGGL((cachegen_cache_kernel<true, false>), grid, block, 0, stream, p);
+  else if (max_half)
+    hipLaunchKernelGGL((cachegen_cache_kernel<false, true>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((cachegen_cache_kernel<false, false>), grid, block, 0, stream, p);
   return check_launch("cachegen_cache_kernel");
 }
 
@@ -929,25 +935,23 @@ int origami_cachegen_unpack_dequantize_to_kv_cache(
   const void* maxes[2] = {max_key, max_value};
 
   if (C % 8 == 0 && aligned16(kv_cache)) {
+    CacheGenCacheParams p{};
     for (int half = 0; half < 2; ++half) {
-      CacheGenCacheParams p{};
-      p.s = make_stream(bytestream + offs[half], lens[half]);
-      p.maxv = maxes[half];
-      p.cache = static_cast<uint16_t*>(kv_cache);
-      p.block_ids = block_ids;
-      p.num_blocks = num_blocks;
-      p.block_count = block_count;
-      p.bs = block_size;
-      p.blk_stride = blk_stride;
-      p.half_stride = half_stride;
-      p.half = half;
-      p.tokens = tokens;
-      p.C = C;
-      p.center = static_cast<float>(bins[half] / 2 - 1);
-      if (int rc = launch_cachegen_cache(p, static_cast<int>(bits[half]), bf16, max_half, st))
-        return rc;
+      p.half[half].s = make_stream(bytestream + offs[half], lens[half]);
+      p.half[half].maxv = maxes[half];
+      p.half[half].bits = static_cast<int32_t>(bits[half]);
+      p.half[half].center = static_cast<float>(bins[half] / 2 - 1);
     }
-    return ORIGAMI_OK;
+    p.cache = static_cast<uint16_t*>(kv_cache);
+    p.block_ids = block_ids;
+    p.num_blocks = num_blocks;
+    p.block_count = block_count;
+    p.bs = block_size;
+    p.blk_stride = blk_stride;
+    p.half_stride = half_stride;
+    p.tokens = tokens;
+    p.C = C;
+    return launch_cachegen_cache(p, bf16, max_half, st);
   }
 
   CacheGenGenericParams p{};
