@@ -428,18 +428,20 @@ def pack_ragged_leg(dev, steps, T=32753, layers=4, H=8, D=128, bs=16):
 
 
 def _staged_pack_kernel(T, H, C, cus):
-    """The staged pack kernel the library picks for T tokens of H heads x C
-    bytes on `cus` CUs (the host rule in set_pack_grid, restated for the
-    label): 16-wave tiles once they give half a tile per CU, single-owner
-    tiles of 1920 tokens when those take no more rounds of tiles per CU."""
+    """The pack kernel the library picks for T tokens (not a multiple of 4) of H
+    heads x C bytes on `cus` CUs (the host rule in set_pack_grid, restated for
+    the label): runs in place with less than half a 16-wave tile per CU or
+    rounds of tiles at most 69% full, else staged 16-wave tiles, single-owner
+    tiles of 1920 tokens when those take no more rounds."""
     cols = 2 * -(-H * C // 128)
     tiles16 = cols * -(-T // 2048)
-    if tiles16 < max(1, cus // 2):
-        return "rows_pack_staged8_kernel (8- or 4-wave tiles; 8-bit runs off 128-byte lines)"
-    if -(-cols * -(-T // 1920) // cus) <= -(-tiles16 // cus):
-        return ("rows_pack_staged8_kernel<16, false, true> (single-owner tiles: each stream "
+    rounds = -(-tiles16 // cus)
+    if tiles16 < max(1, cus // 2) or cols * T / 2048 <= 0.69 * rounds * cus:
+        return "rows_pack_kernel<8, 4> (8-bit runs off 128-byte lines, in place)"
+    if -(-cols * -(-T // 1920) // cus) <= rounds:
+        return ("rows_pack_staged8_kernel<true> (single-owner tiles: each stream "
                 "line written by one tile)")
-    return "rows_pack_staged8_kernel<16, false> (8-bit runs off 128-byte lines)"
+    return "rows_pack_staged8_kernel<false> (8-bit runs off 128-byte lines)"
 
 
 def dequant_leg(src_cache, T, bs, dst_cache, dst_ids, gen, dev, steps, layers=4):
