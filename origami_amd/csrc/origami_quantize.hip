@@ -6,9 +6,12 @@
 // Arithmetic is that of the tensor expressions, operation by operation in binary32
 // without contraction, so payloads are the same bytes: a scalar divided by a tensor is
 // the tensor's reciprocal times the scalar, a tensor divided by a scalar is the tensor
-// times the scalar's reciprocal, and a minimum or maximum with a NaN is a NaN (whose
-// symbols are 0).  The K/V tensor may have any of the layouts the adapters accept: head_dim
-// is its fastest axis, everything else is a stride (KvStrides).
+// times the scalar's reciprocal, and a minimum or maximum with a NaN is that NaN (whose
+// symbols are 0).  One value may have other bytes: the zero point of a KIVI group whose
+// least values are zeros of both signs is -0 here, and there the zero that the reduction's
+// order leaves; both decode to the same values.  The K/V tensor may have any of the layouts
+// the adapters accept: head_dim is its fastest axis, everything else is a stride
+// (KvStrides).
 //
 // HBM bounds both: 4 bytes read and b / 4 bytes written per (K, V) pair of 16-bit
 // values.  16384 tokens of 8 heads x 128, bf16, with the copy of the payload into its
@@ -270,15 +273,13 @@ struct Group {
   float zero, scale, inv;
 };
 
-// `range` holds the minimum (low) and the negated maximum (high); one is a NaN if the
-// other is.
+// `range` holds the minimum (low) and the negated maximum (high).  A NaN keeps its sign and
+// payload through both and through the subtraction, as in the tensor operations.
 __device__ __forceinline__ Group make_group(uint32_t range, float inv_levels) {
   const float tiny = 1.17549435e-38f;  // the least normal binary32
   Group g;
-  const float low = low_half(range);
-  g.zero = low == low ? low : __builtin_nanf("");
-  const float top = low == low ? high_half(range ^ 0x80000000u) : __builtin_nanf("");
-  const float s = __fmul_rn(__fsub_rn(top, g.zero), inv_levels);
+  g.zero = low_half(range);
+  const float s = __fmul_rn(__fsub_rn(high_half(range ^ 0x80000000u), g.zero), inv_levels);
   g.scale = s < tiny ? tiny : s;
   g.inv = __fdiv_rn(1.0f, g.scale);
   return g;

@@ -1,8 +1,9 @@
 """The fused quantizers against the adapters' tensor operations on the same GPU
 tensors, byte for byte: every K/V layout and dtype, rows shorter and longer than a
 wave, symbol runs and planes that do and do not start on words, group sizes the
-kernel does and does not take, ragged token counts, and rows of zeros, infinities
-and NaN."""
+kernel does and does not take, ragged token counts, and rows of zeros of one sign,
+infinities and NaN of either sign and any payload.  The zero point of a KIVI group
+whose least values are zeros of both signs is compared as a value."""
 import pytest
 import torch
 
@@ -99,3 +100,54 @@ def test_unusual_values(cuda_device, dtype, monkeypatch):
     _check_cachegen(kv, {}, 4, monkeypatch)
     for bits in (2, 8):
         _check_kivi(kv, {"bits": bits, "group_size": 64, "sink_tokens": 0}, monkeypatch)
+
+
+def _nan(dtype, sign, payload, dev):
+    """One quiet NaN of the given sign and payload bits (of those float16 keeps)."""
+    bits, width = {torch.bfloat16: (0x7fc0, 16), torch.float16: (0x7e00, 16),
+                   torch.float32: (0x7fc00000, 32)}[dtype]
+    place = {torch.bfloat16: 3, torch.float16: 6, torch.float32: 19}[dtype]
+    v = bits | (payload << place) | (sign << (width - 1))
+    v -= (1 << width) if sign else 0
+    return torch.tensor([v], dtype=torch.int64).to(
+        torch.int16 if width == 16 else torch.int32).view(dtype).to(dev)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("where", ["value", "row", "keys"])
+@pytest.mark.parametrize("sign,payload", [(0, 0), (1, 0), (0, 1), (1, 5)])
+def test_nan_bytes(cuda_device, dtype, where, sign, payload, monkeypatch):
+    kv = _kv(cuda_device, (2, 10, 16, 2, 64), dtype)
+    flat = kv.view(2, 160, 128)
+    nan = _nan(dtype, sign, payload, cuda_device)
+    at = {"value": (slice(None), 60, 7), "row": (slice(None), 61),
+          "keys": (slice(None), slice(64, 128), 9)}[where]
+    flat[at] = nan
+    _check_cachegen(kv, {}, 4, monkeypatch)
+    for bits in (2, 8):
+        _check_kivi(kv, {"bits": bits, "group_size": 64, "sink_tokens": 0}, monkeypatch)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_least_zeros(cuda_device, dtype, monkeypatch):
+    kv = _kv(cuda_device, (2, 10, 16, 2, 64), dtype)
+    flat = kv.view(2, 160, 128)
+    flat[:, :64] = flat[:, :64].abs() + 0.5
+    flat[:, 5, :64] = -0.0  # zeros of one sign in a group
+    flat[:, 6, 64:] = 0.0
+    config = {"bits": 2, "group_size": 64, "sink_tokens": 0}
+    _check_cachegen(kv, {}, 4, monkeypatch)
+    _check_kivi(kv, config, monkeypatch)
+    flat[:, 64:128] = 0.0  # of both signs
+    flat[:, 64:128:2, ::3] = -0.0
+    _check_cachegen(kv, {}, 4, monkeypatch)
+    a = create_quantizer_adapter("kivi", config)
+    q = a.quantize(kv)
+    m, want = q.metadata, a._payload(kv, 0)
+    same = q.symbols == want
+    for name in ("key_zero", "value_zero"):
+        part = slice(m[f"{name}_offset"], m[f"{name}_offset"] + 2 * m[f"{name}_numel"])
+        got, ref = (x[part].view(torch.float16) for x in (q.symbols, want))
+        assert torch.equal(got, ref)  # -0 == 0
+        same[part] = True
+    assert bool(same.all())
