@@ -674,10 +674,21 @@ def _quantize_call(name: str, kv: torch.Tensor, dims: Sequence[int], strides: Se
     return True
 
 
+def _traced(t: torch.Tensor) -> bool:
+    """Whether tensor operations on `t` are recorded, transformed or only
+    propagate shapes: a kernel launched on its address would be left out of
+    the record, or read memory that `t` does not have."""
+    return (type(t) not in (torch.Tensor, torch.nn.Parameter)
+            or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def can_quantize(kv: torch.Tensor) -> bool:
     """Whether `kv` is a tensor the fused quantizers read (their C entry points
     check the rest and return False where they do not apply)."""
-    return kv.is_cuda and kv.dtype in _DTYPE_CODES and kv.is_contiguous() and kv.numel() > 0
+    return (kv.is_cuda and kv.dtype in _DTYPE_CODES and kv.is_contiguous() and kv.numel() > 0
+            and not _traced(kv))
 
 
 def cachegen_quantize(kv: torch.Tensor, *, dims: Sequence[int], strides: Sequence[int],
