@@ -362,6 +362,7 @@ struct CacheGenDenseParams {
   int64_t T, H, D, C;
   int32_t head_groups;    // 8-symbol groups of a head row
   int32_t group_shift;    // log2(head_groups), or -1
+  int64_t tile0;          // first tile of the launch
   CacheGenSegment seg[kDenseSegments];  // blockIdx.y
 };
 
@@ -374,7 +375,7 @@ __device__ __forceinline__ void cachegen_dense_tile(const CacheGenDenseParams& p
                                                     const float* lut) {
   constexpr int NW = (3 + BITS + 3) / 4;
   constexpr uint32_t mask = (1u << BITS) - 1u;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * kDenseTokens;
+  const int64_t t0 = (p.tile0 + blockIdx.x) * kDenseTokens;
   const uint32_t nt = static_cast<uint32_t>(p.T - t0 < kDenseTokens ? p.T - t0 : kDenseTokens);
   const uint32_t GD = p.head_groups;
   const uint32_t items = static_cast<uint32_t>(p.H) * kDenseTokens * GD;
@@ -832,6 +833,9 @@ __global__ __launch_bounds__(kDqThreads) void kivi_generic_kernel(KiviParams p, 
 // Host helpers
 // ---------------------------------------------------------------------------
 
+// Tiles of a launch of the dense restore: a launch holds fewer than 2^32 threads along x.
+constexpr int64_t kMaxDenseTiles = int64_t(1) << 23;
+
 int check_bits(int64_t bits) {
   ORIGAMI_REQUIRE(bits >= 1 && bits <= 8, "Origami CUDA bitpack supports only 1..8 bit symbols");
   return ORIGAMI_OK;
@@ -1018,7 +1022,7 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
   const int64_t tiles = (tokens + kDenseTokens - 1) / kDenseTokens;
   if (head_dim % 8 == 0 && aligned16(output))
     ORIGAMI_REQUIRE(heads <= 65535, "heads exceeds the launch grid");
-  if (head_dim % 8 == 0 && aligned16(output) && C <= (int64_t(1) << 24) && tiles <= INT32_MAX) {
+  if (head_dim % 8 == 0 && aligned16(output) && C <= (int64_t(1) << 24)) {
     CacheGenDenseParams p{};
     p.maxv[0] = max_key;
     p.maxv[1] = max_value;
@@ -1042,12 +1046,14 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
         g.layer = static_cast<int32_t>(layer);
         g.half = static_cast<int32_t>(half);
       }
-      const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(n));
-      if (max_half)
-        hipLaunchKernelGGL((cachegen_dense_kernel<true>), grid, dim3(kDqThreads), 0, st, p);
-      else
-        hipLaunchKernelGGL((cachegen_dense_kernel<false>), grid, dim3(kDqThreads), 0, st, p);
-      if (int rc = check_launch("cachegen_dense_kernel")) return rc;
+      for (p.tile0 = 0; p.tile0 < tiles; p.tile0 += kMaxDenseTiles) {
+        const dim3 grid(grid_for(tiles - p.tile0, 1, kMaxDenseTiles), static_cast<unsigned>(n));
+        if (max_half)
+          hipLaunchKernelGGL((cachegen_dense_kernel<true>), grid, dim3(kDqThreads), 0, st, p);
+        else
+          hipLaunchKernelGGL((cachegen_dense_kernel<false>), grid, dim3(kDqThreads), 0, st, p);
+        if (int rc = check_launch("cachegen_dense_kernel")) return rc;
+      }
     }
     return ORIGAMI_OK;
   }
