@@ -353,7 +353,7 @@ struct CacheGenSegment {
 };
 
 constexpr int kDenseSegments = 32;   // segments of a launch (kernel arguments)
-constexpr int kDenseTokens = 16;     // tokens of a tile, all heads
+constexpr int kDenseShift = 4;       // log2 of a tile's tokens, all heads (dense_token_shift)
 constexpr int kDenseBatch = 4;       // groups a thread loads before expanding
 
 struct CacheGenDenseParams {
@@ -362,23 +362,26 @@ struct CacheGenDenseParams {
   int64_t T, H, D, C;
   int32_t head_groups;    // 8-symbol groups of a head row
   int32_t group_shift;    // log2(head_groups), or -1
+  int32_t token_shift;    // log2(tokens of a tile)
   int64_t tile0;          // first tile of the launch
   CacheGenSegment seg[kDenseSegments];  // blockIdx.y
 };
 
-// A tile of kDenseTokens tokens x all heads, D % 8 == 0: a thread takes 8-symbol groups
+// A tile of 2^token_shift tokens x all heads, D % 8 == 0: a thread takes 8-symbol groups
 // in the order of the output (head, token, dim), so a wave writes whole runs of one
 // head's rows (1 KiB at D = 128) and the tile reads a contiguous stretch of the stream.
-template <int BITS, bool MAX_HALF>
+template <int BITS, bool MAX_HALF, int SHIFT>
 __device__ __forceinline__ void cachegen_dense_tile(const CacheGenDenseParams& p,
                                                     const CacheGenSegment& seg,
                                                     const float* lut) {
   constexpr int NW = (3 + BITS + 3) / 4;
   constexpr uint32_t mask = (1u << BITS) - 1u;
-  const int64_t t0 = (p.tile0 + blockIdx.x) * kDenseTokens;
-  const uint32_t nt = static_cast<uint32_t>(p.T - t0 < kDenseTokens ? p.T - t0 : kDenseTokens);
+  const int shift = SHIFT >= 0 ? SHIFT : p.token_shift;
+  const uint32_t tile_tokens = 1u << shift;
+  const int64_t t0 = (p.tile0 + blockIdx.x) << shift;
+  const uint32_t nt = static_cast<uint32_t>(p.T - t0 < tile_tokens ? p.T - t0 : tile_tokens);
   const uint32_t GD = p.head_groups;
-  const uint32_t items = static_cast<uint32_t>(p.H) * kDenseTokens * GD;
+  const uint32_t items = (static_cast<uint32_t>(p.H) << shift) * GD;
   const uint32_t G = static_cast<uint32_t>(p.C >> 3);
   const int64_t row0 = static_cast<int64_t>(seg.layer) * p.T + t0;
   uint16_t* const out =
@@ -392,8 +395,8 @@ __device__ __forceinline__ void cachegen_dense_tile(const CacheGenDenseParams& p
       const uint32_t i = i0 + j * kDqThreads;
       const uint32_t row = p.group_shift >= 0 ? i >> p.group_shift : i / GD;
       dg[j] = i - row * GD;
-      tt[j] = row % kDenseTokens;
-      hh[j] = row / kDenseTokens;
+      tt[j] = row & (tile_tokens - 1);
+      hh[j] = row >> shift;
       w[j][0] = w[j][1] = w[j][2] = 0;
       mraw[j] = 0;
       o[j] = 0;
@@ -442,7 +445,8 @@ __device__ __forceinline__ void cachegen_dense_tile(const CacheGenDenseParams& p
 // All segments in one launch (blockIdx.y).  One launch per segment with the heads as
 // grid rows, 8 times the stream's reads, took 46.8 us for 4 layers of 8192 tokens of
 // 8 heads x 128; this takes 26.2 us (a copy of as many bytes 32.9).
-template <bool MAX_HALF>
+// SHIFT: log2 of a tile's tokens, or -1 where p.token_shift holds it.
+template <bool MAX_HALF, int SHIFT>
 __global__ __launch_bounds__(kDqThreads) void cachegen_dense_kernel(CacheGenDenseParams p) {
   __shared__ float lut[256];
   const CacheGenSegment& seg = p.seg[blockIdx.y];
@@ -450,14 +454,14 @@ __global__ __launch_bounds__(kDqThreads) void cachegen_dense_kernel(CacheGenDens
     lut[i] = cachegen_level(i, seg.center);
   __syncthreads();
   switch (seg.bits) {
-    case 1: return cachegen_dense_tile<1, MAX_HALF>(p, seg, lut);
-    case 2: return cachegen_dense_tile<2, MAX_HALF>(p, seg, lut);
-    case 3: return cachegen_dense_tile<3, MAX_HALF>(p, seg, lut);
-    case 4: return cachegen_dense_tile<4, MAX_HALF>(p, seg, lut);
-    case 5: return cachegen_dense_tile<5, MAX_HALF>(p, seg, lut);
-    case 6: return cachegen_dense_tile<6, MAX_HALF>(p, seg, lut);
-    case 7: return cachegen_dense_tile<7, MAX_HALF>(p, seg, lut);
-    default: return cachegen_dense_tile<8, MAX_HALF>(p, seg, lut);
+    case 1: return cachegen_dense_tile<1, MAX_HALF, SHIFT>(p, seg, lut);
+    case 2: return cachegen_dense_tile<2, MAX_HALF, SHIFT>(p, seg, lut);
+    case 3: return cachegen_dense_tile<3, MAX_HALF, SHIFT>(p, seg, lut);
+    case 4: return cachegen_dense_tile<4, MAX_HALF, SHIFT>(p, seg, lut);
+    case 5: return cachegen_dense_tile<5, MAX_HALF, SHIFT>(p, seg, lut);
+    case 6: return cachegen_dense_tile<6, MAX_HALF, SHIFT>(p, seg, lut);
+    case 7: return cachegen_dense_tile<7, MAX_HALF, SHIFT>(p, seg, lut);
+    default: return cachegen_dense_tile<8, MAX_HALF, SHIFT>(p, seg, lut);
   }
 }
 
@@ -836,6 +840,19 @@ __global__ __launch_bounds__(kDqThreads) void kivi_generic_kernel(KiviParams p, 
 // Tiles of a launch of the dense restore: a launch holds fewer than 2^32 threads along x.
 constexpr int64_t kMaxDenseTiles = int64_t(1) << 23;
 
+// log2 of the tokens of a dense restore's tile: 16, or fewer, while every thread keeps a
+// group, where those leave less than three tiles per CU.  us for 8 heads x 128, one
+// layer, with 16 / 8 / 4 / 2 tokens: 100 tokens 6.1 / 4.1 / 3.3 / 2.9, 1000 6.4 / 4.5 /
+// 3.8 / 3.8, 2000 6.5 / 4.7 / 4.3 / 4.9, 4096 6.9 / 5.7 / 5.9 / 7.2, 8192 8.6 / 8.0 / 9.2 /
+// 11.6; 1 head x 64, 1000 tokens 2.80 / 2.78 / 2.93 / 3.25.
+int dense_token_shift(int64_t tokens, int64_t C, int64_t segments) {
+  int shift = kDenseShift;
+  while (shift > 0 && ((tokens + (int64_t(1) << shift) - 1) >> shift) * segments < 768 &&
+         (C << (shift - 1)) / 8 >= kDqThreads)
+    --shift;
+  return shift;
+}
+
 int check_bits(int64_t bits) {
   ORIGAMI_REQUIRE(bits >= 1 && bits <= 8, "Origami CUDA bitpack supports only 1..8 bit symbols");
   return ORIGAMI_OK;
@@ -1019,7 +1036,6 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool max_half = max_dtype == ORIGAMI_DTYPE_FLOAT16;
   const size_t esize = max_half ? 2 : 4;
-  const int64_t tiles = (tokens + kDenseTokens - 1) / kDenseTokens;
   if (head_dim % 8 == 0 && aligned16(output))
     ORIGAMI_REQUIRE(heads <= 65535, "heads exceeds the launch grid");
   if (head_dim % 8 == 0 && aligned16(output) && C <= (int64_t(1) << 24)) {
@@ -1035,6 +1051,9 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
     p.group_shift = -1;
     for (int i = 0; i < 22; ++i)
       if (p.head_groups == 1 << i) p.group_shift = i;
+    const int64_t most = 2 * layers < kDenseSegments ? 2 * layers : kDenseSegments;
+    p.token_shift = dense_token_shift(tokens, C, most);
+    const int64_t tiles = (tokens + (int64_t(1) << p.token_shift) - 1) >> p.token_shift;
     for (int64_t j0 = 0; j0 < 2 * layers; j0 += kDenseSegments) {
       const int64_t n = 2 * layers - j0 < kDenseSegments ? 2 * layers - j0 : kDenseSegments;
       for (int64_t k = 0; k < n; ++k) {
@@ -1047,11 +1066,16 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
         g.half = static_cast<int32_t>(half);
       }
       for (p.tile0 = 0; p.tile0 < tiles; p.tile0 += kMaxDenseTiles) {
-        const dim3 grid(grid_for(tiles - p.tile0, 1, kMaxDenseTiles), static_cast<unsigned>(n));
-        if (max_half)
-          hipLaunchKernelGGL((cachegen_dense_kernel<true>), grid, dim3(kDqThreads), 0, st, p);
+        const dim3 grid(grid_for(tiles - p.tile0, 1, kMaxDenseTiles), static_cast<unsigned>(n)),
+            block(kDqThreads);
+        if (max_half && p.token_shift == kDenseShift)
+          hipLaunchKernelGGL((cachegen_dense_kernel<true, kDenseShift>), grid, block, 0, st, p);
+        else if (max_half)
+          hipLaunchKernelGGL((cachegen_dense_kernel<true, -1>), grid, block, 0, st, p);
+        else if (p.token_shift == kDenseShift)
+          hipLaunchKernelGGL((cachegen_dense_kernel<false, kDenseShift>), grid, block, 0, st, p);
         else
-          hipLaunchKernelGGL((cachegen_dense_kernel<false>), grid, dim3(kDqThreads), 0, st, p);
+          hipLaunchKernelGGL((cachegen_dense_kernel<false, -1>), grid, block, 0, st, p);
         if (int rc = check_launch("cachegen_dense_kernel")) return rc;
       }
     }
