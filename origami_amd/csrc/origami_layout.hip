@@ -660,9 +660,10 @@ struct LanePlanes {
 // belong to no symbol that is kept.  Its loads go out with the others; loading such a run
 // again, guarded dword by dword, after the others had returned made the one wave that
 // holds the stream's end a serial chain.
-template <int NW>
+// WINDOW: the last dword of a window run holds bytes of the run, so no run passes the end.
+template <int NW, bool WINDOW>
 __device__ __forceinline__ void load_run(const RowsParams& p, int64_t byte0, uint32_t* w) {
-  if (byte0 + 4 * NW <= p.stream_bytes) {
+  if (WINDOW || byte0 + 4 * NW <= p.stream_bytes) {
     if constexpr (NW == 5) {
       load_run_dwords<4>(p.stream + byte0, w);
       load_run_dwords<1>(p.stream + byte0 + 16, w + 4);
@@ -703,6 +704,10 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlane
 #pragma unroll
     for (int i = 0; i < NU; ++i)
       u[i] = __builtin_amdgcn_alignbit(i + 1 < NW ? w[i + 1] : 0u, w[i], sh);
+    if constexpr (!SERIAL && MODE == kRowsWindow && BITS == 3) {
+#pragma unroll
+      for (int i = 0; i < NU; ++i) asm volatile("" : "+v"(u[i]));
+    }
     expand16<BITS>(u, out);
   };
   if constexpr (SERIAL) {
@@ -713,7 +718,7 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlane
       if (d < 0 || !any) continue;
       const int64_t P = d + p.bit_bias + sym0 * BITS;
       uint32_t w[NW];
-      load_run<NW>(p, first_byte(P), w);
+      load_run<NW, MODE == kRowsWindow>(p, first_byte(P), w);
       expand(w, funnel(P), v[k]);
     }
   } else {
@@ -759,14 +764,21 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlane
         if (d >= 0 && any) {
           const int64_t P = d + p.bit_bias + sym0 * BITS;
           shp[k >> 2] |= funnel(P) << (8 * (k & 3));
-          load_run<NW>(p, first_byte(P), w[k]);
+          load_run<NW, MODE == kRowsWindow>(p, first_byte(P), w[k]);
         }
       }
     }
-    // every plane's dwords are requested before any is used
+    // Every plane's dwords are requested before any is used.  Left to itself the compiler
+    // carries the shifted dwords of 3- and 7-bit windows to the transposition (102 and 134
+    // registers; 83-88 and 97-104 with each plane's finished here, one more wave per SIMD:
+    // 7-bit batch of 8 x 8192 tokens 47.6 -> 44.5 us).
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int k = 0; k < 16; ++k) expand(w[k], (shp[k >> 2] >> (8 * (k & 3))) & 31u, v[k]);
+    for (int k = 0; k < 16; ++k) {
+      expand(w[k], (shp[k >> 2] >> (8 * (k & 3))) & 31u, v[k]);
+      if constexpr (MODE == kRowsWindow && BITS == 7)
+        asm volatile("" : "+v"(v[k][0]), "+v"(v[k][1]), "+v"(v[k][2]), "+v"(v[k][3]));
+    }
   }
 }
 
@@ -1074,15 +1086,18 @@ __device__ __forceinline__ int64_t cursor_row(const RowsParams& p, int half, con
 // HBM peak) and launches of few waves per CU up to half their time, while
 // whole-tile launches of 8 or more waves per CU run 1-4% faster with it: the
 // host picks by launch size (waves_per_cu).
-// SHORT: all 16 rows without a check each where the lane has them (launches of few waves
-// per CU; the split restores are 0.5% faster with the checks between their stores).
-template <bool ONEBLK, bool SHORT, class F>
+// WHOLE: all 16 rows without a check each where the lane has them.  Only the single-request
+// shift restores take it (2053 tokens x 8 heads, 5 bits 8.8 -> 8.0 us; 4104 tokens 7.9 ->
+// 7.4): elsewhere the second copy of the rows costs 20-45 registers and scratch memory (a
+// batch of 4 x 2048 tokens, 8 bits 8.9 us with it and 7.5 without, packs of 4096 tokens at 2
+// bits 8.6 and 7.7, of 8192 at 4 bits 13.8 and 12.5).
+template <bool ONEBLK, bool WHOLE = false, class F>
 __device__ __forceinline__ void for_rows16(const RowsParams& p, int half, RowCursor rc,
                                            int64_t nrows, F&& f) {
   if constexpr (ONEBLK) {
     const int64_t row0 = cursor_row(p, half, rc);
     if (row0 < 0) return;
-    if (SHORT && nrows >= 16) {
+    if (WHOLE && nrows >= 16) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) f(j, row0 + j);
     } else {
@@ -1106,7 +1121,8 @@ __device__ __forceinline__ void for_rows16(const RowsParams& p, int half, RowCur
 // Rows kernels
 // ---------------------------------------------------------------------------
 
-template <int BITS, int MODE, bool SPLIT = false, bool ONEBLK = false, bool SERIAL = false>
+template <int BITS, int MODE, bool SPLIT = false, bool ONEBLK = false, bool SERIAL = false,
+          bool WHOLE = false>
 __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
                                             const int64_t* desc, int slice = 0) {
   const TileCoord tc = tile_coord<SPLIT>(p, ti, slice);
@@ -1115,11 +1131,13 @@ __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
   const int64_t sym0 = static_cast<int64_t>(tc.half) * p.T + tc.t0;
 
   constexpr bool kShort = ONEBLK && !SPLIT;
+  // the batched shift restores at 7 and 8 bits have no registers left for it
+  constexpr bool kEarlyCursor = kShort && (WHOLE || MODE != kRowsShift);
   RowCursor rc;
-  if constexpr (kShort) cursor_init(p, tc.t0, rc);
+  if constexpr (kEarlyCursor) cursor_init(p, tc.t0, rc);
   uint32_t v[16][4];
   load_planes16<BITS, MODE, SERIAL>(p, lane_planes<kShort>(p, tc, desc), sym0, nv > 0, v);
-  if constexpr (!kShort) cursor_init(p, tc.t0, rc);
+  if constexpr (!kEarlyCursor) cursor_init(p, tc.t0, rc);
   if (MODE == kRowsShift && nv < 16) {  // other modes: T % 16 == 0
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
@@ -1136,7 +1154,7 @@ __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
 
   uint8_t* col = p.rows + static_cast<int64_t>(tc.h) * p.head_pitch + tc.q * 16;
   // each row is written once: non-temporal
-  for_rows16<ONEBLK, kShort>(p, tc.half, rc, p.row_tokens - tc.t0, [&](int j, int64_t row) {
+  for_rows16<ONEBLK, WHOLE>(p, tc.half, rc, p.row_tokens - tc.t0, [&](int j, int64_t row) {
     const u32x4 x = {o[j][0], o[j][1], o[j][2], o[j][3]};
     __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(col + row * p.row_pitch));
   });
@@ -1150,7 +1168,7 @@ __global__ __launch_bounds__(kRowsThreads) void rows_unpack_kernel(RowsParams p)
   for (int64_t tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
     const TileIndex ti = split_tile(p, tile);
     if (!ONEBLK || p.planes) load_descriptors(p, ti, desc);
-    unpack_tile<BITS, MODE, false, ONEBLK, SERIAL>(p, ti, desc);
+    unpack_tile<BITS, MODE, false, ONEBLK, SERIAL, ONEBLK && MODE == kRowsShift>(p, ti, desc);
   }
 }
 
@@ -1226,7 +1244,7 @@ __device__ __forceinline__ void unpack_tile_wide(const RowsParams& p, TileIndex 
     transpose16(v, o);
     RowCursor rc;
     cursor_init(p, t0, rc);
-    for_rows16<ONEBLK, ONEBLK>(p, tc.half, rc, p.row_tokens - t0, [&](int j, int64_t row) {
+    for_rows16<ONEBLK>(p, tc.half, rc, p.row_tokens - t0, [&](int j, int64_t row) {
       const u32x4 x = {o[j][0], o[j][1], o[j][2], o[j][3]};
       __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(col + row * p.row_pitch));
     });
@@ -1370,7 +1388,7 @@ __device__ __forceinline__ void load_tile_rows(const RowsParams& p, const TileCo
   if (nv <= 0) return;
   RowCursor rc;
   cursor_init(p, tc.t0, rc);
-  for_rows16<ONEBLK, ONEBLK>(p, tc.half, rc, nv, [&](int j, int64_t row) {
+  for_rows16<ONEBLK>(p, tc.half, rc, nv, [&](int j, int64_t row) {
     const u32x4 x =
         __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(col + row * p.row_pitch));
     r[j][0] = x.x;
