@@ -1982,16 +1982,18 @@ void set_divisors(RowsParams& p) {
 }
 
 // Waves of a tile in a launch of fewer than two 4-wave tiles per CU, `units` wave tiles
-// of work: 2 or 1 where they lower the most waves a CU gets (tiles per CU rounded up,
-// less 5% of a CU, times waves per tile) by enough to pay for the shorter runs.  Restore
+// of work: 2 or 1 where they lower the most waves a CU gets (tiles per CU rounded up, in
+// restores less 5% of a CU, times waves per tile) by enough to pay for the shorter runs.  Restore
 // of Llama-3-8B geometry, us with 4 / 2 / 1 waves: 1024 tokens 5.99 / 4.56 / 3.93, 2176
 // 6.24 / 6.74 / 5.87, 4096 7.27 / 8.54 / 7.54, 4104 9.20 / 10.32 / 10.23, 5001 14.3 /
 // 14.7 / 11.6, 6144 14.4 / 13.2 / 13.0, 7168 14.0 / 16.1 / 14.5; pack 1024 tokens 6.48 /
-// 5.63 / 5.20, 4096 8.21 / 8.14 / 8.87, 5120 12.5 / 9.9 / 9.4, 7168 13.1 / 13.3 / 12.0.
+// 5.63 / 5.20, 4096 8.21 / 8.14 / 8.87, 5120 12.5 / 9.9 / 9.4, 7168 13.1 / 13.3 / 12.0;
+// off the dwords, where a pack's tiles are long, 4104 tokens 5 bits 20.7 / 17.9 / 17.5, 2053
+// tokens 7 bits 38.7 / 38.3 / 34.8.
 int short_tile_waves(double units, bool pack) {
   const double cus = device_cu_count();
   auto load = [&](int waves) {
-    return std::max(1.0, std::ceil((units - 0.05 * cus) / (cus * waves))) * waves;
+    return std::max(1.0, std::ceil((units - (pack ? 0 : 0.05 * cus)) / (cus * waves))) * waves;
   };
   int best = 4;
   for (int waves = 2; waves >= 1; waves /= 2)
@@ -2039,7 +2041,14 @@ void set_grid_dims(RowsParams& p, int64_t H, int64_t C, int64_t tile_tokens_tota
   // more.
   if (tiles < want && waves == 4 && wq_max != 1) {
     const double units = static_cast<double>(nhalf * H * nqg) * segs / kLaneSegs;
-    tiles = shape(short_tile_waves(units, pack));
+    waves = short_tile_waves(units, pack);
+    // A 1-wave tile with 3 or 4 of its 8 token runs: restores in wide runs 11.3 us in 2-wave
+    // tiles, 12.7 in 1-wave ones (192 and 256 tokens, 2 bits; with 1 or 2 runs 18.7 / 13.3),
+    // 4-bit packs of 64 tokens 5.7 / 5.9.
+    const int64_t last = segs % kLaneSegs;
+    if ((last == 3 || last == 4) && (seg_tokens != kSegTokens || (pack && segs < kLaneSegs)))
+      waves = std::max(waves, 2);
+    tiles = shape(waves);
   }
   const int64_t segs_per_wg = static_cast<int64_t>(p.ws) * kLaneSegs;
   p.partial_last = p.nst > 1 && segs % segs_per_wg != 0;
