@@ -7,7 +7,7 @@
 // Both directions move each byte once, so HBM bounds them.  A lane owns 16 (or 32)
 // consecutive symbols, so symbol accesses are 16 bytes per lane and a wave covers
 // 1 KiB; the packed side is the lane's 2b (4b) bytes, adjacent to its neighbours'.
-// Large launches keep kRunUnroll groups in flight per lane.
+// Large unpacks keep kRunUnroll groups in flight per lane.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -20,10 +20,13 @@ using namespace origami_internal;
 namespace {
 
 constexpr int kRunThreads = 256;
-// Groups of one lane in flight, kRunThreads apart: 4 when the launch has at least
-// kRunUnrollGroups groups (two workgroups per CU of 4 groups per lane), else 1.
+// Groups of one lane in flight in the unpack, kRunThreads apart: 4 when the launch has at
+// least kRunUnrollGroups groups, else 1.  us with 1 / 4, 5-bit symbols not in a cache: 8.4M
+// 4.3 / 5.3, 16.8M 6.4 / 6.1, 33.6M 10.2 / 9.7, 67M 17.8 / 17.4, 134M 32.7 / 32.8 (8 bits:
+// 4.6 / 4.4, 6.8 / 7.1, 12.2 / 11.8, 21.6 / 20.7, 45.1 / 46.5).  The pack keeps 1: 8.4M 4.7 /
+// 5.6, 33.6M 12.7 / 13.6, 134M 40.3 / 42.7.
 constexpr int kRunUnroll = 4;
-constexpr int64_t kRunUnrollGroups = int64_t(2) * 256 * kRunThreads * kRunUnroll;
+constexpr int64_t kRunUnrollGroups = int64_t(1) << 20;
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
@@ -78,15 +81,29 @@ __device__ __forceinline__ void store_dwords(uint8_t* dst, const uint32_t* w) {
   }
 }
 
-// Symbol i of a run whose first symbol is at bit `bit0` of the stream.
+// The symbols of group s .. s + 15 that lie in [0, count), one byte each: a run's first
+// or last group, or one whose dwords pass the end of the stream.  Its loads go out
+// together (symbol by symbol, two loads and a store each in turn, a stream of 100 5-bit
+// symbols took 5.2 us; now 3.5).
 template <int BITS>
-__device__ __forceinline__ uint8_t run_symbol(const RunParams& p, int64_t bit0, int64_t i) {
-  const int64_t bit = bit0 + i * BITS;
+__device__ __forceinline__ void unpack_part(const RunParams& p, int64_t bit0, int64_t s,
+                                            int64_t count, uint8_t* out) {
+  constexpr int NU = (16 * BITS + 31) / 32;
+  const int64_t bit = bit0 + s * BITS;  // negative before a stream's first symbol
   const int64_t byte = (bit >> 5) * 4;
-  const uint32_t lo = load_dword_guarded(p.stream, byte, p.stream_bytes);
-  const uint32_t hi = load_dword_guarded(p.stream, byte + 4, p.stream_bytes);
-  return static_cast<uint8_t>(
-      __builtin_amdgcn_alignbit(hi, lo, static_cast<uint32_t>(bit & 31)) & ((1u << BITS) - 1u));
+  uint32_t w[NU + 1], x[NU > 4 ? NU : 4], o[4];
+#pragma unroll
+  for (int i = 0; i <= NU; ++i) {
+    const int64_t at = byte + 4 * i;
+    w[i] = at < 0 ? 0 : load_dword_guarded(p.stream, at, p.stream_bytes);
+  }
+#pragma unroll
+  for (int i = 0; i < NU; ++i)
+    x[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], static_cast<uint32_t>(bit & 31));
+  expand16<BITS>(x, o);
+#pragma unroll
+  for (int j = 0; j < 16; ++j)
+    if (s + j >= 0 && s + j < count) out[s + j] = static_cast<uint8_t>(o[j >> 2] >> (8 * (j & 3)));
 }
 
 // Stream -> symbols.  Group g holds the 16 symbols whose bytes are the g-th aligned
@@ -128,9 +145,8 @@ __global__ __launch_bounds__(kRunThreads) void runs_unpack_kernel(RunParams p) {
         expand16<BITS>(x, o);
         __builtin_nontemporal_store(u32x4{o[0], o[1], o[2], o[3]},
                                     reinterpret_cast<u32x4*>(out + s));
-      } else {  // a run's first or last group, or the end of the stream
-        for (int64_t i = s < 0 ? 0 : s; i < s + 16 && i < r.count; ++i)
-          out[i] = run_symbol<BITS>(p, bit0, i);
+      } else if (s < r.count) {
+        unpack_part<BITS>(p, bit0, s, r.count, out);
       }
     }
   }
@@ -140,57 +156,42 @@ __global__ __launch_bounds__(kRunThreads) void runs_unpack_kernel(RunParams p) {
 // for even b, 32 for odd), so lanes never share a dword; the run's last group, if it
 // is not whole, is written byte by byte with zero pad bits.  The run's symbols and
 // its stream bytes start on dwords.
-template <int BITS, int U>
+template <int BITS>
 __global__ __launch_bounds__(kRunThreads) void runs_pack_kernel(RunParams p) {
   constexpr int GS = BITS % 2 == 0 ? 16 : 32, NV = GS / 16, ND = GS * BITS / 32;
   const SymbolRun r = p.run[blockIdx.y];
   const uint8_t* const src = p.symbols + r.symbol;
   uint8_t* const dst = p.flat + r.byte;
   const int64_t groups = (r.count + GS - 1) / GS;
-  const int64_t step = static_cast<int64_t>(gridDim.x) * kRunThreads * U;
-  for (int64_t g0 = (static_cast<int64_t>(blockIdx.x) * U) * kRunThreads + threadIdx.x;
-       g0 < groups; g0 += step) {
-    uint32_t w[U][NV][4];
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kRunThreads;
+  for (int64_t g = static_cast<int64_t>(blockIdx.x) * kRunThreads + threadIdx.x; g < groups;
+       g += step) {
+    const int64_t s = g * GS;
+    const bool whole = s + GS <= r.count;
+    uint32_t w[NV][4];
+    if (whole) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t s = (g0 + u * kRunThreads) * GS;
-      if (s + GS <= r.count) {
+      for (int v = 0; v < NV; ++v) load_dwords<4>(src + s + 16 * v, w[v]);
+    } else {  // the run's last symbols, zeros past them, all loads in flight together
 #pragma unroll
-        for (int v = 0; v < NV; ++v) load_dwords<4>(src + s + 16 * v, w[u][v]);
-      } else {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) w[u][v][0] = w[u][v][1] = w[u][v][2] = w[u][v][3] = 0;
-      }
+      for (int q = 0; q < GS / 4; ++q) w[q >> 2][q & 3] = load_dword_guarded(src, s + 4 * q, r.count);
     }
+    uint32_t d[ND] = {};
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t s = (g0 + u * kRunThreads) * GS;
-      if (s + GS <= r.count) {
-        uint32_t d[ND] = {};
+    for (int j = 0; j < GS; ++j) {
+      const uint32_t sym = (w[j >> 4][(j >> 2) & 3] >> (8 * (j & 3))) & ((1u << BITS) - 1u);
+      const int dw = (j * BITS) >> 5, off = (j * BITS) & 31;
+      d[dw] |= sym << off;
+      if (off + BITS > 32) d[dw + 1] |= sym >> (32 - off);
+    }
+    uint8_t* const o = dst + g * (4 * ND);
+    if (whole) {
+      store_dwords<ND>(o, d);
+    } else {
+      const int n = static_cast<int>(((r.count - s) * BITS + 7) >> 3);
 #pragma unroll
-        for (int j = 0; j < GS; ++j) {
-          const uint32_t sym =
-              (w[u][j >> 4][(j >> 2) & 3] >> (8 * (j & 3))) & ((1u << BITS) - 1u);
-          const int dw = (j * BITS) >> 5, off = (j * BITS) & 31;
-          d[dw] |= sym << off;
-          if (off + BITS > 32) d[dw + 1] |= sym >> (32 - off);
-        }
-        store_dwords<ND>(dst + s / GS * (4 * ND), d);
-      } else if (s < r.count) {
-        uint8_t* o = dst + s / GS * (4 * ND);
-        uint32_t acc = 0;
-        int n = 0;
-        for (int64_t i = s; i < r.count; ++i) {
-          acc |= (src[i] & ((1u << BITS) - 1u)) << n;
-          n += BITS;
-          if (n >= 8) {
-            *o++ = static_cast<uint8_t>(acc);
-            acc >>= 8;
-            n -= 8;
-          }
-        }
-        if (n > 0) *o = static_cast<uint8_t>(acc);
-      }
+      for (int i = 0; i < 4 * ND; ++i)
+        if (i < n) o[i] = static_cast<uint8_t>(d[i >> 2] >> (8 * (i & 3)));
     }
   }
 }
@@ -220,12 +221,8 @@ template <int BITS>
 int launch_pack(const RunParams& p, int nrun, int64_t symbols, hipStream_t stream) {
   constexpr int GS = BITS % 2 == 0 ? 16 : 32;
   const int64_t groups = (symbols + GS - 1) / GS;
-  const bool many = groups * nrun >= kRunUnrollGroups;
-  const dim3 grid(grid_for(groups, int64_t(kRunThreads) * (many ? kRunUnroll : 1), 65536), nrun);
-  if (many)
-    hipLaunchKernelGGL((runs_pack_kernel<BITS, kRunUnroll>), grid, dim3(kRunThreads), 0, stream, p);
-  else
-    hipLaunchKernelGGL((runs_pack_kernel<BITS, 1>), grid, dim3(kRunThreads), 0, stream, p);
+  const dim3 grid(grid_for(groups, kRunThreads, 65536), nrun);
+  hipLaunchKernelGGL((runs_pack_kernel<BITS>), grid, dim3(kRunThreads), 0, stream, p);
   return check_launch("runs_pack_kernel");
 }
 
