@@ -210,16 +210,19 @@ int launch_cachegen(const CacheGenQuantParams& p, hipStream_t stream) {
   return check_launch("cachegen_quantize_kernel");
 }
 
-// Groups per lane by row length (at most 4096 channels), and several row steps in
-// flight where the launch still gives every CU two workgroups.
+// Groups per lane by row length (at most 4096 channels), and several row steps in flight
+// per wave in long launches.  us with 1 / 4 steps, bf16 not in a cache: 8 heads x 128, 4096
+// tokens 7.4 / 9.0, 8192 12.0 / 12.8, 12288 16.7 / 16.9, 16384 20.6 / 20.0, 32768 36.8 /
+// 33.6; 4 x 128, 6144 tokens 7.2 / 7.6, 8192 8.8 / 8.6, 16384 15.3 / 13.4; 2 x 64, 24576
+// tokens 7.0 / 7.3, 32768 8.5 / 8.0.
 template <int DT>
 int launch_cachegen_rows(const CacheGenQuantParams& p, hipStream_t stream) {
   const int64_t steps = (static_cast<int64_t>(p.tokens) * p.row_lanes / 64) * 2 / kQWaves;
   if (p.groups <= 64)
-    return steps >= 4 * 512 ? launch_cachegen<DT, 1, 4>(p, stream)
+    return steps >= 4096 ? launch_cachegen<DT, 1, 4>(p, stream)
                             : launch_cachegen<DT, 1, 1>(p, stream);
   if (p.groups <= 128)
-    return steps >= 4 * 512 ? launch_cachegen<DT, 2, 4>(p, stream)
+    return steps >= 8192 ? launch_cachegen<DT, 2, 4>(p, stream)
                             : launch_cachegen<DT, 2, 1>(p, stream);
   if (p.groups <= 256) return launch_cachegen<DT, 4, 1>(p, stream);
   return launch_cachegen<DT, 8, 1>(p, stream);
