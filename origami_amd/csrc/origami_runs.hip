@@ -7,7 +7,7 @@
 // Both directions move each byte once, so HBM bounds them.  A lane owns 16 (or 32)
 // consecutive symbols, so symbol accesses are 16 bytes per lane and a wave covers
 // 1 KiB; the packed side is the lane's 2b (4b) bytes, adjacent to its neighbours'.
-// Large unpacks keep kRunUnroll groups in flight per lane.
+// Large unpacks and 8-bit packs keep kRunUnroll groups in flight per lane.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -20,11 +20,13 @@ using namespace origami_internal;
 namespace {
 
 constexpr int kRunThreads = 256;
-// Groups of one lane in flight in the unpack, kRunThreads apart: 4 when the launch has at
-// least kRunUnrollGroups groups, else 1.  us with 1 / 4, 5-bit symbols not in a cache: 8.4M
-// 4.3 / 5.3, 16.8M 6.4 / 6.1, 33.6M 10.2 / 9.7, 67M 17.8 / 17.4, 134M 32.7 / 32.8 (8 bits:
-// 4.6 / 4.4, 6.8 / 7.1, 12.2 / 11.8, 21.6 / 20.7, 45.1 / 46.5).  The pack keeps 1: 8.4M 4.7 /
-// 5.6, 33.6M 12.7 / 13.6, 134M 40.3 / 42.7.
+// Groups of one lane in flight in the unpack and the 8-bit pack (the copy of a payload into
+// its chunks), kRunThreads apart: 4 when the launch has at least kRunUnrollGroups groups,
+// else 1.  us with 1 / 4, 5-bit symbols not in a cache: 8.4M 4.3 / 5.3, 16.8M 6.4 / 6.1,
+// 33.6M 10.2 / 9.7, 67M 17.8 / 17.4, 134M 32.7 / 32.8 (8 bits: 4.6 / 4.4, 6.8 / 7.1, 12.2 /
+// 11.8, 21.6 / 20.7, 45.1 / 46.5).  CacheGen saves, whose payload was just written: 10.6 MB
+// 18.4 / 20.3, 21 MB 28.6 / 27.0, 42 MB 46.4 / 45.5.  The other packs keep 1: 5 bits, 8.4M
+// 4.7 / 5.6, 33.6M 12.7 / 13.6, 134M 40.3 / 42.7.
 constexpr int kRunUnroll = 4;
 constexpr int64_t kRunUnrollGroups = int64_t(1) << 20;
 
@@ -84,7 +86,7 @@ __device__ __forceinline__ void store_dwords(uint8_t* dst, const uint32_t* w) {
 // The symbols of group s .. s + 15 that lie in [0, count), one byte each: a run's first
 // or last group, or one whose dwords pass the end of the stream.  Its loads go out
 // together (symbol by symbol, two loads and a store each in turn, a stream of 100 5-bit
-// symbols took 5.2 us; now 3.5).
+// symbols took 5.2 us; now 2.6).
 template <int BITS>
 __device__ __forceinline__ void unpack_part(const RunParams& p, int64_t bit0, int64_t s,
                                             int64_t count, uint8_t* out) {
@@ -156,42 +158,50 @@ __global__ __launch_bounds__(kRunThreads) void runs_unpack_kernel(RunParams p) {
 // for even b, 32 for odd), so lanes never share a dword; the run's last group, if it
 // is not whole, is written byte by byte with zero pad bits.  The run's symbols and
 // its stream bytes start on dwords.
-template <int BITS>
+template <int BITS, int U>
 __global__ __launch_bounds__(kRunThreads) void runs_pack_kernel(RunParams p) {
   constexpr int GS = BITS % 2 == 0 ? 16 : 32, NV = GS / 16, ND = GS * BITS / 32;
   const SymbolRun r = p.run[blockIdx.y];
   const uint8_t* const src = p.symbols + r.symbol;
   uint8_t* const dst = p.flat + r.byte;
   const int64_t groups = (r.count + GS - 1) / GS;
-  const int64_t step = static_cast<int64_t>(gridDim.x) * kRunThreads;
-  for (int64_t g = static_cast<int64_t>(blockIdx.x) * kRunThreads + threadIdx.x; g < groups;
-       g += step) {
-    const int64_t s = g * GS;
-    const bool whole = s + GS <= r.count;
-    uint32_t w[NV][4];
-    if (whole) {
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kRunThreads * U;
+  for (int64_t g0 = (static_cast<int64_t>(blockIdx.x) * U) * kRunThreads + threadIdx.x; g0 < groups;
+       g0 += step) {
+    uint32_t w[U][NV][4];
 #pragma unroll
-      for (int v = 0; v < NV; ++v) load_dwords<4>(src + s + 16 * v, w[v]);
-    } else {  // the run's last symbols, zeros past them, all loads in flight together
+    for (int u = 0; u < U; ++u) {
+      const int64_t s = (g0 + u * kRunThreads) * GS;
+      if (s + GS <= r.count) {
 #pragma unroll
-      for (int q = 0; q < GS / 4; ++q) w[q >> 2][q & 3] = load_dword_guarded(src, s + 4 * q, r.count);
+        for (int v = 0; v < NV; ++v) load_dwords<4>(src + s + 16 * v, w[u][v]);
+      } else {  // the run's last symbols, zeros past them, all loads in flight together
+#pragma unroll
+        for (int q = 0; q < GS / 4; ++q)
+          w[u][q >> 2][q & 3] = load_dword_guarded(src, s + 4 * q, r.count);
+      }
     }
-    uint32_t d[ND] = {};
 #pragma unroll
-    for (int j = 0; j < GS; ++j) {
-      const uint32_t sym = (w[j >> 4][(j >> 2) & 3] >> (8 * (j & 3))) & ((1u << BITS) - 1u);
-      const int dw = (j * BITS) >> 5, off = (j * BITS) & 31;
-      d[dw] |= sym << off;
-      if (off + BITS > 32) d[dw + 1] |= sym >> (32 - off);
-    }
-    uint8_t* const o = dst + g * (4 * ND);
-    if (whole) {
-      store_dwords<ND>(o, d);
-    } else {
-      const int n = static_cast<int>(((r.count - s) * BITS + 7) >> 3);
+    for (int u = 0; u < U; ++u) {
+      const int64_t s = (g0 + u * kRunThreads) * GS;
+      if (s >= r.count) continue;
+      uint32_t d[ND] = {};
 #pragma unroll
-      for (int i = 0; i < 4 * ND; ++i)
-        if (i < n) o[i] = static_cast<uint8_t>(d[i >> 2] >> (8 * (i & 3)));
+      for (int j = 0; j < GS; ++j) {
+        const uint32_t sym = (w[u][j >> 4][(j >> 2) & 3] >> (8 * (j & 3))) & ((1u << BITS) - 1u);
+        const int dw = (j * BITS) >> 5, off = (j * BITS) & 31;
+        d[dw] |= sym << off;
+        if (off + BITS > 32) d[dw + 1] |= sym >> (32 - off);
+      }
+      uint8_t* const o = dst + s / GS * (4 * ND);
+      if (s + GS <= r.count) {
+        store_dwords<ND>(o, d);
+      } else {
+        const int n = static_cast<int>(((r.count - s) * BITS + 7) >> 3);
+#pragma unroll
+        for (int i = 0; i < 4 * ND; ++i)
+          if (i < n) o[i] = static_cast<uint8_t>(d[i >> 2] >> (8 * (i & 3)));
+      }
     }
   }
 }
@@ -221,8 +231,16 @@ template <int BITS>
 int launch_pack(const RunParams& p, int nrun, int64_t symbols, hipStream_t stream) {
   constexpr int GS = BITS % 2 == 0 ? 16 : 32;
   const int64_t groups = (symbols + GS - 1) / GS;
-  const dim3 grid(grid_for(groups, kRunThreads, 65536), nrun);
-  hipLaunchKernelGGL((runs_pack_kernel<BITS>), grid, dim3(kRunThreads), 0, stream, p);
+  const bool many = BITS == 8 && groups * nrun >= kRunUnrollGroups;
+  const dim3 grid(grid_for(groups, int64_t(kRunThreads) * (many ? kRunUnroll : 1), 65536), nrun),
+      block(kRunThreads);
+  if constexpr (BITS == 8) {
+    if (many) {
+      hipLaunchKernelGGL((runs_pack_kernel<8, kRunUnroll>), grid, block, 0, stream, p);
+      return check_launch("runs_pack_kernel");
+    }
+  }
+  hipLaunchKernelGGL((runs_pack_kernel<BITS, 1>), grid, block, 0, stream, p);
   return check_launch("runs_pack_kernel");
 }
 
