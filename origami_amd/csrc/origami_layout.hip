@@ -415,6 +415,7 @@ constexpr int kThreads = 256;          // generic and block-copy kernels
 // bandwidth, so idle CUs cost more than short runs.
 constexpr int kRowsMaxWaves = 16;
 constexpr int kRowsThreads = kRowsMaxWaves * 64;  // launch bound
+constexpr int kOneBlockMaxWaves = 4;              // of one-block restores (one_block_rows)
 // A restore launch with at least kRowsSplitTiles tiles per CU dispatches each
 // tile as waves / kRowsSplitWaves workgroups of kRowsSplitWaves waves, each a
 // column of wave tiles along tokens (same tile geometry and order).  Per layer:
@@ -1086,11 +1087,13 @@ __device__ __forceinline__ int64_t cursor_row(const RowsParams& p, int half, con
 // HBM peak) and launches of few waves per CU up to half their time, while
 // whole-tile launches of 8 or more waves per CU run 1-4% faster with it: the
 // host picks by launch size (waves_per_cu).
-// WHOLE: all 16 rows without a check each where the lane has them.  Only the single-request
-// shift restores take it (2053 tokens x 8 heads, 5 bits 8.8 -> 8.0 us; 4104 tokens 7.9 ->
-// 7.4): elsewhere the second copy of the rows costs 20-45 registers and scratch memory (a
-// batch of 4 x 2048 tokens, 8 bits 8.9 us with it and 7.5 without, packs of 4096 tokens at 2
-// bits 8.6 and 7.7, of 8192 at 4 bits 13.8 and 12.5).
+// WHOLE: all 16 rows without a check each where the lane has them.  The single-request shift
+// and 8-bit aligned restores take it (2053 tokens x 8 heads, 5 bits 8.8 -> 8.0 us; 4104
+// tokens 7.9 -> 7.4; 16 tokens, 8 bits 3.5 -> 3.1), in kernels bounded at their 4 waves, for
+// which the second copy of the rows needs no scratch memory.  Elsewhere it costs 20-45
+// registers: window restores of 4-9 MB of K/V 7%, a batch of 4 x 2048 tokens at 8 bits 8.9
+// us with it and 7.5 without, packs of 4096 tokens at 2 bits 8.6 and 7.7, of 8192 at 4 bits
+// 13.8 and 12.5.
 template <bool ONEBLK, bool WHOLE = false, class F>
 __device__ __forceinline__ void for_rows16(const RowsParams& p, int half, RowCursor rc,
                                            int64_t nrows, F&& f) {
@@ -1163,12 +1166,14 @@ __device__ __forceinline__ void unpack_tile(const RowsParams& p, TileIndex ti,
 // ONEBLK as for for_rows16, SERIAL as for load_planes16; the host picks both
 // by launch size.
 template <int BITS, int MODE, bool ONEBLK, bool SERIAL>
-__global__ __launch_bounds__(kRowsThreads) void rows_unpack_kernel(RowsParams p) {
+__global__
+__launch_bounds__(ONEBLK ? kOneBlockMaxWaves * 64 : kRowsThreads) void rows_unpack_kernel(
+    RowsParams p) {
   __shared__ int64_t desc[kTilePlanes];
   for (int64_t tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
     const TileIndex ti = split_tile(p, tile);
     if (!ONEBLK || p.planes) load_descriptors(p, ti, desc);
-    unpack_tile<BITS, MODE, false, ONEBLK, SERIAL, ONEBLK && MODE == kRowsShift>(p, ti, desc);
+    unpack_tile<BITS, MODE, false, ONEBLK, SERIAL, ONEBLK && MODE != kRowsWindow>(p, ti, desc);
   }
 }
 
@@ -2128,7 +2133,8 @@ double waves_per_cu(int64_t ntiles, int waves) {
   return w < 16.0 ? w : 16.0;
 }
 
-// Row order of the whole-tile row kernels by launch size (waves per CU).
+// Row order of the whole-tile row kernels by launch size (waves per CU).  Restores of at
+// most 6 waves per CU have tiles of at most kOneBlockMaxWaves waves (set_grid_dims).
 // One-block rows (for_rows16) for restores up to 6 waves per CU (4096 tokens of
 // Llama-3-8B: 9.6 -> 8.0 us; 8192 tokens: 14.0 -> 14.6, so not above), for packs up to 12 (4096 tokens: 2.07 -> 4.03 TB/s;
 // 12288: 4.50 -> 4.74; 16384 tokens at 16: 5.07 -> 4.83).  Serial plane loads
@@ -2432,7 +2438,8 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
   const double wpc = waves_per_cu(p.ntiles, p.waves);
   const bool staged = mode == kRowsStaged8;
   const bool oneblk =
-      one_block_rows(p) && wpc <= (pack ? kOneBlockPackWaves : kOneBlockWaves);
+      one_block_rows(p) && wpc <= (pack ? kOneBlockPackWaves : kOneBlockWaves) &&
+      (pack || p.waves <= kOneBlockMaxWaves);
   const bool serial = wpc > kSerialLoadWaves;
   if (mode == kRowsWide || mode == kRowsWideCached) {
     if (pack || p.waves > kWideMaxWaves)
