@@ -161,6 +161,10 @@ __global__ __launch_bounds__(kRunThreads) void runs_unpack_kernel(RunParams p) {
 template <int BITS, int U>
 __global__ __launch_bounds__(kRunThreads) void runs_pack_kernel(RunParams p) {
   constexpr int GS = BITS % 2 == 0 ? 16 : 32, NV = GS / 16, ND = GS * BITS / 32;
+  // The last group of odd widths, up to 31 symbols, is loaded together and packed like the
+  // others: 10007 7-bit symbols 4.6 -> 3.0 us.  Up to 15 symbols go one by one: as fast, and
+  // the kernels of even widths are 2-5% faster with the shorter code (4.2M symbols 2.9 -> 2.75).
+  constexpr bool kWholeTail = BITS % 2 == 1;
   const SymbolRun r = p.run[blockIdx.y];
   const uint8_t* const src = p.symbols + r.symbol;
   uint8_t* const dst = p.flat + r.byte;
@@ -175,16 +179,32 @@ __global__ __launch_bounds__(kRunThreads) void runs_pack_kernel(RunParams p) {
       if (s + GS <= r.count) {
 #pragma unroll
         for (int v = 0; v < NV; ++v) load_dwords<4>(src + s + 16 * v, w[u][v]);
-      } else {  // the run's last symbols, zeros past them, all loads in flight together
+      } else {  // the run's last symbols, zeros past them
 #pragma unroll
         for (int q = 0; q < GS / 4; ++q)
-          w[u][q >> 2][q & 3] = load_dword_guarded(src, s + 4 * q, r.count);
+          w[u][q >> 2][q & 3] = kWholeTail ? load_dword_guarded(src, s + 4 * q, r.count) : 0;
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t s = (g0 + u * kRunThreads) * GS;
       if (s >= r.count) continue;
+      if (!kWholeTail && s + GS > r.count) {
+        uint8_t* o = dst + s / GS * (4 * ND);
+        uint32_t acc = 0;
+        int n = 0;
+        for (int64_t i = s; i < r.count; ++i) {
+          acc |= (src[i] & ((1u << BITS) - 1u)) << n;
+          n += BITS;
+          if (n >= 8) {
+            *o++ = static_cast<uint8_t>(acc);
+            acc >>= 8;
+            n -= 8;
+          }
+        }
+        if (n > 0) *o = static_cast<uint8_t>(acc);
+        continue;
+      }
       uint32_t d[ND] = {};
 #pragma unroll
       for (int j = 0; j < GS; ++j) {
