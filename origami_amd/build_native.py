@@ -14,7 +14,7 @@ from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 REPO = PKG.parent
-SOURCES = [PKG / "csrc" / f"origami_{name}.hip" 
+SOURCES = [PKG / "csrc" / f"origami_{name}.hip"
            for name in ("layout", "dequant", "runs", "quantize")]
 INCLUDE = REPO / "include"
 LIB_DIR = PKG / "_lib"

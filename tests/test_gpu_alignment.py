@@ -36,20 +36,20 @@ def _oracle_threads():
 
 
 @pytest.mark.parametrize("T", [
-    32784,   # planes 32 bytes off the line (2T % 128 == 32), 33 token tiles
+    32784,   # planes 32 bytes off the line (2T % 128 == 32): runs written in place
     32832,   # planes on lines, V half 64 bytes off
     32896,   # planes and V half on lines, 128-token partial last tile
-    40000,   # planes 64 bytes off, partial last tile
+    40000,   # planes on lines, V half 64 bytes off, partial last tile
     49216,   # planes on lines, V half off, partial last tile
-    3088,    # small: 4-wave tiles, partial last tile
+    3088,    # small: tiles of few waves, partial last tile
     32753,   # odd: runs at any byte; staged pack in 16-wave tiles, non-temporal stores
     65521,   # odd: staged pack at 4 tiles per CU, plain stores
     12001,   # odd: staged pack, each stream line written by one tile (1 round)
     24001,   # the same over 2 rounds of tiles
     49217,   # the same over 4 rounds of tiles
     16383,   # odd: staged pack in 16-wave tiles, one per CU
-    4100,    # staged pack in 8-wave tiles, 4-token last tile
-    2053,    # staged pack in 4-wave tiles
+    4100,    # runs on dwords written in place, 4-token last run
+    2053,    # odd and short: runs written in place at any byte
 ])
 @pytest.mark.parametrize("blocks_first", [False, True])
 def test_byte_planes_off_lines(cuda_device, T, blocks_first):
@@ -127,10 +127,11 @@ def test_staged_pack_into_offset_stream(cuda_device, shift, T):
 
 @pytest.mark.parametrize("seed", range(12))
 def test_staged_pack_random_geometries(cuda_device, seed):
-    """Seeded staged packs at 5000-60000 odd token counts, 2-8 heads of 128
-    or 256 bytes, block sizes 8, 16, 24 or 32, both cache layouts and an output
-    pointer 0-64 bytes into its buffer.  Most of these draws take 16-wave
-    tiles in which each stream line is written by one tile.  The stream
+    """Seeded packs off 128-byte lines at 5000-60000 odd token counts, 2-8 heads
+    of 128 or 256 bytes, block sizes 8, 16, 24 or 32, both cache layouts and an
+    output pointer 0-64 bytes into its buffer.  On 256 CUs half of these draws
+    take staged tiles in which each stream line is written by one tile, half
+    write their runs in place.  The stream
     equals the oracle's and the bytes around it keep their guard value."""
     dev = cuda_device
     rng = np.random.default_rng(900 + seed)

@@ -45,8 +45,7 @@ def _check(dev, T, H, D, shift, bs=16, blocks_first=False, seed=0):
     (0, 1, 8, 0), (0, 1, 64, 1), (16, 1, 128, 16), (112, 2, 64, 3), (256, 1, 128, 0),
     (768, 2, 128, 5), (2048, 4, 128, 0)])
 def test_every_remainder(cuda_device, tokens, heads, head_dim, shift, rest):
-    if tokens + rest:
-        _check(cuda_device, tokens + rest, heads, head_dim, shift, blocks_first=rest % 2 == 1)
+    _check(cuda_device, tokens + rest or 48, heads, head_dim, shift, blocks_first=rest % 2 == 1)
 
 
 @pytest.mark.parametrize("tokens,shift", [
