@@ -661,10 +661,9 @@ struct LanePlanes {
 // belong to no symbol that is kept.  Its loads go out with the others; loading such a run
 // again, guarded dword by dword, after the others had returned made the one wave that
 // holds the stream's end a serial chain.
-// WINDOW: the last dword of a window run holds bytes of the run, so no run passes the end.
-template <int NW, bool WINDOW>
+template <int NW>
 __device__ __forceinline__ void load_run(const RowsParams& p, int64_t byte0, uint32_t* w) {
-  if (WINDOW || byte0 + 4 * NW <= p.stream_bytes) {
+  if (byte0 + 4 * NW <= p.stream_bytes) {
     if constexpr (NW == 5) {
       load_run_dwords<4>(p.stream + byte0, w);
       load_run_dwords<1>(p.stream + byte0 + 16, w + 4);
@@ -719,7 +718,7 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlane
       if (d < 0 || !any) continue;
       const int64_t P = d + p.bit_bias + sym0 * BITS;
       uint32_t w[NW];
-      load_run<NW, MODE == kRowsWindow>(p, first_byte(P), w);
+      load_run<NW>(p, first_byte(P), w);
       expand(w, funnel(P), v[k]);
     }
   } else {
@@ -765,19 +764,21 @@ __device__ __forceinline__ void load_runs16(const RowsParams& p, const LanePlane
         if (d >= 0 && any) {
           const int64_t P = d + p.bit_bias + sym0 * BITS;
           shp[k >> 2] |= funnel(P) << (8 * (k & 3));
-          load_run<NW, MODE == kRowsWindow>(p, first_byte(P), w[k]);
+          load_run<NW>(p, first_byte(P), w[k]);
         }
       }
     }
     // Every plane's dwords are requested before any is used.  Left to itself the compiler
-    // carries the shifted dwords of 3- and 7-bit windows to the transposition (102 and 134
-    // registers; 83-88 and 97-104 with each plane's finished here, one more wave per SIMD:
-    // 7-bit batch of 8 x 8192 tokens 47.6 -> 44.5 us).
+    // carries the dwords of 3-, 5-, 6- and 7-bit windows to the transposition.  With the
+    // shifts (3 bits) or the symbols (5 to 7) finished here a wave more fits a SIMD: 3 bits
+    // 102 -> 88 registers, 5 bits 111 -> 96, 7 bits 134 -> 104.  us per layer of 32768 tokens,
+    // not in a cache: 5 bits 51.6 -> 48.8, 6 bits 53.1 -> 49.8, 7 bits 59.9 -> 54.4.  5- and
+    // 6-bit launches of few waves per CU are slower so (4096 tokens 9.2, 8.5 without).
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       expand(w[k], (shp[k >> 2] >> (8 * (k & 3))) & 31u, v[k]);
-      if constexpr (MODE == kRowsWindow && BITS == 7)
+      if constexpr (MODE == kRowsWindow && (BITS == 7 || (!CLOSED && (BITS == 5 || BITS == 6))))
         asm volatile("" : "+v"(v[k][0]), "+v"(v[k][1]), "+v"(v[k][2]), "+v"(v[k][3]));
     }
   }
