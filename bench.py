@@ -483,7 +483,7 @@ def dequant_leg(src_cache, T, bs, dst_cache, dst_ids, gen, dev, steps, layers=4)
         if name == "cachegen":
             read = (m["key_stream_bytes"] + m["value_stream_bytes"]
                     + 2 * (m["key_max_numel"] + m["value_max_numel"]))
-            kernel = "cachegen_cache_kernel<4, bf16, f16 max>"
+            kernel = "cachegen_cache_kernel<bf16, f16 max> (4 bits, both halves)"
         else:
             read = (m["key_stream_bytes"] + m["value_stream_bytes"]
                     + 2 * sum(m[f"{k}_numel"] for k in ("key_scale", "key_zero", "value_scale",
@@ -523,7 +523,7 @@ def dequant_leg(src_cache, T, bs, dst_cache, dst_ids, gen, dev, steps, layers=4)
 
 def _cachegen_dense_leg(T, H, D, dev, steps, layers):
     """CacheGen unpack + dequantize into the float16 [layers, 2, H, T, D]
-    tensor (cachegen_dense_kernel, one launch per K or V stream segment):
+    tensor (cachegen_dense_kernel, all stream segments in one launch):
     `layers` layers at 4-bit keys and values, 16 bins, float16 per-token
     maxima.  The streams are zeros, so every value must come out as minus
     its token's maximum (symbol 0 dequantizes to (0 - c) / c * max, c = 7),
@@ -563,7 +563,7 @@ def _cachegen_dense_leg(T, H, D, dev, steps, layers):
     ms = e0.elapsed_time(e1) / (steps * layers)
     alg = 2 * seg + 2 * T * 2 + 2 * H * T * D * 2
     gbps = alg / (ms * 1e-3) / 1e9
-    return {"kernel": "cachegen_dense_kernel<4> (float16 [L, 2, H, T, D] output)",
+    return {"kernel": "cachegen_dense_kernel<f16 max, 16 tokens> (float16 [L, 2, H, T, D] output)",
             "bits": [4, 4], "layers": layers, "per_layer_us": round(ms * 1e3, 2),
             "algorithmic_bytes_per_layer": int(alg), "gbps": round(gbps, 2),
             "frac": round(gbps / HBM_PEAK_GBPS, 4), "output_ok": ok}

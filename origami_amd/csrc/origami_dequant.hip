@@ -1036,6 +1036,7 @@ int origami_cachegen_unpack_dequantize(const uint8_t* bytestream, int64_t bytest
   const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool max_half = max_dtype == ORIGAMI_DTYPE_FLOAT16;
   const size_t esize = max_half ? 2 : 4;
+  // No kernel here needs the limit; calls beyond it have always been refused.
   if (head_dim % 8 == 0 && aligned16(output))
     ORIGAMI_REQUIRE(heads <= 65535, "heads exceeds the launch grid");
   if (head_dim % 8 == 0 && aligned16(output) && C <= (int64_t(1) << 24)) {

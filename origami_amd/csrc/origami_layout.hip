@@ -510,7 +510,7 @@ struct RowsParams {
   int32_t H;
   int32_t nq;                // C / 16
   int32_t waves;             // waves per workgroup (16, 8, 4, 2 or 1)
-  int32_t wq;                // wave tiles along channels per workgroup (1, 2, 4)
+  int32_t wq;                // wave tiles along channels per workgroup (1 or 2)
   int32_t ws;                // wave tiles along tokens per workgroup (waves / wq)
   int32_t nqt;               // workgroups along channels
   int32_t nst;               // workgroups along tokens
@@ -1341,9 +1341,11 @@ __global__ __launch_bounds__(kRowsSplitWaves * 64) void rows_unpack_batch_split_
   __shared__ int64_t desc[kTilePlanes];
   const int64_t slots = b.common.ntiles << sh;
   for (int64_t i = blockIdx.x; i < slots; i += gridDim.x) {
-    // pairs of slices, which share stream lines off 128-byte lines, on one XCD: the
-    // 8-request Qwen2.5-7B batch 135.2 us with runs of 1, 134.0 of 2, 134.5 of 4, 135.0
-    // of 16
+    // Pairs of slices, which share stream lines, on one XCD.  us with runs of 1 / 2 / 4
+    // slices, 256-byte heads: 3 bits, 4 x 32768 tokens x 8 heads 127 / 118 / -, 5 bits, the
+    // same x 4 heads 75.5 / 71.2 / 70.8, 4 bits, 8 ragged requests x 4 heads 91.6 / 86.7 /
+    // 87.1.  Aligned 4-bit batches lose up to 2%, at 8 bits the three are within 2% (4
+    // heads, 8 ragged requests 213.9 / 213.6 / 214.0).
     const int64_t s = xcd_run_order(i, slots, 2);
     batch_tile<BITS, MODE, true, ONEBLK, false>(b, s >> sh, desc,
                                                static_cast<int>(s & ((1 << sh) - 1)));
@@ -2268,11 +2270,11 @@ void set_restore_grid(RowsParams& p, int mode, int bits, int64_t H, int64_t C,
     set_grid_dims(p, H, C, tile_tokens_total, nhalf);
 }
 
-// Mode of the rows pack: 8-bit planes off 128-byte lines go through LDS so
-// that every stream line is written whole (32753 tokens: 3062 -> 3766 GB/s;
-// 32784, planes 32 bytes off: 3163 -> 3399).  Planes on lines keep in-place
-// non-temporal stores even when the V half is not: 3874 against 3608 staged
-// at 32832 tokens.
+// Mode of the rows pack.  For 8-bit planes off 128-byte lines it proposes the staged
+// pack, which writes stream lines whole through LDS (32753 tokens: 3062 -> 3766 GB/s);
+// set_pack_grid decides between it and runs written in place.  Planes on lines keep
+// in-place non-temporal stores even when the V half is not: 3874 against 3608 staged at
+// 32832 tokens.
 int pack_mode(const PlanInfo& info, const RowsParams& p, int64_t T) {
   if (info.bits < 8 && (!info.byte_aligned || (T * info.bits) % 8 != 0)) return kRowsBits;
   const int mode = rows_mode(info, p, T, true);
@@ -2481,8 +2483,7 @@ int launch_rows(bool pack, const RowsParams& params, int64_t nhalf, int bits, in
   if (staged) {
     if (!pack || bits != 8) return fail(ORIGAMI_ERR_INVALID, "staged rows mode is the 8-bit pack");
     // Non-temporal chunk stores below kStagedNtTiles tiles per CU.  Pack
-    // GB/s, plain -> non-temporal (same box, two runs each): 4100 tokens
-    // 1696 / 1697 -> 1802 / 1762, 8199: 2368 / 2366 -> 2584 / 2606, 16383:
+    // GB/s, plain -> non-temporal (same box, two runs each): 16383 tokens
     // 4429 / 4375 -> 4637 / 4795, 32753: 4292 / 4303 -> 4308 / 4333, 49217:
     // 3638 / 3645 -> 3766 / 3776; 65521 tokens (4 tiles per CU): 4203 / 4201
     // -> 4135 / 4119.

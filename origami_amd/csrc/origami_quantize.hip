@@ -13,9 +13,9 @@
 // the adapters accept: head_dim is its fastest axis, everything else is a stride
 // (KvStrides).
 //
-// HBM bounds both: 4 bytes read and b / 4 bytes written per (K, V) pair of 16-bit
-// values.  16384 tokens of 8 heads x 128, bf16, with the copy of the payload into its
-// stored chunks: CacheGen 573 -> 26.7 us, KIVI (2 bits) 1025 -> 30.1 us.
+// HBM bounds CacheGen, its own arithmetic KIVI; 4 bytes are read and b / 4 bytes written
+// per (K, V) pair of 16-bit values.  16384 tokens of 8 heads x 128, bf16, with the copy of
+// the payload into its stored chunks: CacheGen 573 -> 26.7 us, KIVI (2 bits) 1025 -> 30.0 us.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -251,9 +251,8 @@ struct KiviQuantParams {
 
 constexpr int kQTokens = 16;  // tokens of a lane
 
-// Two float16 values per register: the ranges are taken on pairs.
-// The least and greatest of three, NaN if one is a NaN (gfx950's IEEE 754-2019 minimum
-// and maximum).
+// The ranges are taken on pairs, two float16 values per register: the least and the
+// greatest of three, NaN if one is a NaN (gfx950's IEEE 754-2019 minimum and maximum).
 __device__ __forceinline__ uint32_t pk_min3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t r;
   asm("v_pk_minimum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -385,8 +384,9 @@ __device__ __forceinline__ void each(F&& f) {
 // division and symbols gathered by fused multiply-adds took the save of 16384 tokens
 // from 61.0 us (scalar ranges, a branch per quotient, shifts) to 33.3; ranges by the
 // three-operand minimum and maximum, which carry NaNs, the subtraction of the zero point
-// folded into the conversion and one address per lane to 30.1.  A cap of 96 registers
-// for five waves per SIMD spills (58 us).
+// folded into the conversion and one address per lane to 30.1.  It runs three waves per
+// SIMD at 164-172 registers (two at 8 bits of bfloat16); a cap at four waves spills 58-69 of
+// them, one at five waves took 58 us.
 template <int HALF, int DT, int W, bool BYTES>
 __device__ __forceinline__ void kivi_quantize_tile(const KiviQuantParams& p, uint32_t tile) {
   constexpr int CL = HALF == 0 ? 8 : 16, TL = 64 / CL;  // lanes along channels, tokens

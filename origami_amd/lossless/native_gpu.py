@@ -551,7 +551,7 @@ def cachegen_unpack_dequantize_to_kv_cache(
     """CacheGen fused restore into the paged cache (native_gpu.py:178-215,
     bitpack_layout_cuda.cpp:475-581): the K and V streams are unpacked,
     dequantized ((s - c) / c * max[token]) and written to the listed blocks
-    in one kernel per half.  Tokens >= `tokens` are left untouched."""
+    in one launch.  Tokens >= `tokens` are left untouched."""
     flat = bytestream.reshape(-1)
     if not flat.is_contiguous():
         flat = flat.contiguous()
